@@ -232,6 +232,8 @@ struct DenseIdxBwdParams {
 int launch_dense_scores_bwd(const DenseIdxBwdParams& p, hipStream_t stream);
 
 int launch_sparse_mla_fwd(const SparseFwdParams& p, hipStream_t stream);
+// n_heads <= 64 (dsa_sparse_fwd_fh.hip); called by launch_sparse_mla_fwd
+int launch_sparse_mla_fwd_fh(const SparseFwdParams& p, hipStream_t stream);
 // ev (nullable): 6 events recorded around the stages B4 | B1 | B2 | B3 | B5.
 int launch_sparse_mla_bwd(const SparseBwdParams& p, hipStream_t stream, hipEvent_t const* ev);
 // B3 with int8 G rows (p.g_int8), launched by launch_sparse_mla_bwd.

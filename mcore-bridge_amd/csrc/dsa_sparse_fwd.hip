@@ -444,22 +444,12 @@ int launch_sparse_mla_fwd(const SparseFwdParams& p, hipStream_t stream) {
   if (p.split_keys > kMaxTopk || p.n_split < 1 || (p.n_split > 1 && p.split_keys % kBK != 0)) return -2;
   if ((int64_t)(p.n_split - 1) * p.split_keys >= p.topk) return -1;   // every split owns >= 1 slot
   if (p.sinks != nullptr && p.n_split != 1) return -2;                  // a sink joins each row once
+  if (p.n_heads <= 64) return launch_sparse_mla_fwd_fh(p, stream);
   const dim3 grid(xcd_grid(p.total_q * p.n_split, p.n_xcd), (p.n_heads + 127) / 128);
-  const int nw = p.n_heads > 64 ? 4 : (p.n_heads > 32 ? 2 : 1);
-  if (p.q_dim == kDv) {   // 512-wide q: the rope-free instantiation
-    if (nw == 4)
-      hipLaunchKernelGGL((sparse_mla_fwd_kernel<4, false>), grid, dim3(256), 0, stream, p);
-    else if (nw == 2)
-      hipLaunchKernelGGL((sparse_mla_fwd_kernel<2, false>), grid, dim3(128), 0, stream, p);
-    else
-      hipLaunchKernelGGL((sparse_mla_fwd_kernel<1, false>), grid, dim3(64), 0, stream, p);
-  } else if (nw == 4) {
+  if (p.q_dim == kDv)   // 512-wide q: the rope-free instantiation
+    hipLaunchKernelGGL((sparse_mla_fwd_kernel<4, false>), grid, dim3(256), 0, stream, p);
+  else
     hipLaunchKernelGGL((sparse_mla_fwd_kernel<4, true>), grid, dim3(256), 0, stream, p);
-  } else if (nw == 2) {
-    hipLaunchKernelGGL((sparse_mla_fwd_kernel<2, true>), grid, dim3(128), 0, stream, p);
-  } else {
-    hipLaunchKernelGGL((sparse_mla_fwd_kernel<1, true>), grid, dim3(64), 0, stream, p);
-  }
   return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
