@@ -272,12 +272,10 @@ __global__ __launch_bounds__(NW * 64, 1) void bwd_sp_kernel(SparseBwdParams p) {
 }
 
 // ------------------------------------------------------------------------------------------
-// B2: dQ^T[576 x 32*NW heads] = K^T . (scale*dS)^T over the query's gathered rows, with
-// 16x16x32 MFMAs.  Wave w owns 576/NW latent dims (DT tiles of 16) for every head of the
-// workgroup (HT tiles of 16): per 32-key block it reads DT K^T fragments (transposing reads of
-// the KV tile) and HT dS^T fragments, each K^T fragment feeding HT MFMAs and each dS^T fragment
-// DT.  (Split by heads instead, every wave would read the whole K^T tile for 36 MFMAs: four
-// times the LDS reads.)
+// B2: dQ^T[576 x 128 heads] = K^T . (scale*dS)^T over the query's gathered rows, with 16x16x32
+// MFMAs (64 < n_heads <= 128).  The latent dims are split over the waves, every wave covering all
+// heads: K^T fragments (transposing reads of the KV tile) are read once per workgroup.  (Split by
+// heads instead, every wave would read the whole K^T tile for 36 MFMAs: four times the LDS reads.)
 // ------------------------------------------------------------------------------------------
 constexpr int kDsTileBytes = 128 * 64;  // [128 heads][32 keys] bf16
 constexpr int kDqPitch = kDqk * 2 + 16;  // LDS pitch of a staged bf16 dQ row
@@ -294,158 +292,7 @@ struct DqSmem {
   int red[8];
 };
 
-template <int NW, bool ROPE>
-__global__ __launch_bounds__(NW * 64, 1) void bwd_dq_kernel(SparseBwdParams p) {
-  constexpr int DQ = ROPE ? kDqk : kDv;                        // dq row width
-  constexpr int HR = 32 * NW;                                  // head rows of the workgroup
-  constexpr int HT = HR / 16;                                  // head tiles
-  constexpr int DT = DQ / 16 / NW;                             // dim tiles per wave
-  constexpr int TC = tile_copies_per_wave<NW, ROPE>();
-  constexpr int G = TC + HR / 16 / NW;
-  static_assert(HR / 16 / NW == 2, "two dS copies per wave per block");
-  static_assert(DT * NW * 16 == DQ && DT >= TC, "dims split evenly; one tile copy per dim step");
-  __shared__ __attribute__((aligned(128))) DqSmem sm;
-  const int t = xcd_remap(blockIdx.x, p.n_xcd);
-  if (t >= p.total_q) return;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int g = lane >> 4, gi = lane & 15;
-  const int h0 = blockIdx.y * 128;
-  const int nblk = stage_index_row<NW>(sm.idx, sm.red, p.idx + (int64_t)t * p.idx_stride, p.topk, p.n_kv,
-                                       p.causal, t + p.q_offset);
-  // dS rows of this workgroup's heads; rows past n_heads re-read row 0 (never stored).
-  const int hrows = min(HR, p.n_heads - h0);
-  // staged dS tile of block b: [H heads][32 keys] contiguous at ((t * NB + b) * H) * 32
-  const char* ds_base = reinterpret_cast<const char*>(p.ds_stage + ((int64_t)t * (p.topk_pad / kBK) * p.n_heads + h0) * kBK);
-  const int64_t ds_blk = (int64_t)p.n_heads * kBK * 2;   // bytes per staged block tile
-  // copy k (0 <= k < 2) of this wave's share of block blk's dS rows
-  auto copy_ds_part = [&](char* dst, int blk, int k) {
-    const uint32_t base = __builtin_amdgcn_readfirstlane(lds_addr(dst));
-    const int w = __builtin_amdgcn_readfirstlane(wave);
-    const int i = w + k * NW;
-    const int h = 16 * i + (lane >> 2);
-    const int q = (lane & 3) ^ ((h >> 1) & 3);
-    const int hs = h < hrows ? h : 0;
-    async_copy16_nt(ds_base + blk * ds_blk + hs * (kBK * 2) + q * 16, base + i * 1024u);
-  };
-  auto copy_ds = [&](char* dst, int blk) {
-#pragma unroll
-    for (int k = 0; k < HR / 16 / NW; ++k) copy_ds_part(dst, blk, k);
-  };
-
-  // A operand (K^T, dims x keys) of dim tile D: lane (g, gi) gets dim 16D + gi, keys 8g .. 8g+7
-  // as two transposing reads of 4 keys (rows 8g + gi/4 and 8g + 4 + gi/4, 4 dims from
-  // 16D + 4(gi%4)).  V dims (D < 32): tile row key_row(key) (keys 8g + j sit 2 rows apart:
-  // conflict-free), byte kv[h] + 32D; rope dims: kr[h] ^ (32(D - 32)).
-  uint32_t kv[2], kr[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const uint32_t key = 8 * g + 4 * h + (gi >> 2);
-    kv[h] = key_row(key) * kTileVPitch + 8u * (gi & 3);
-    kr[h] = kTileVBytes + key * 128u + 8u * (gi & 1) + 16u * (((gi & 3) >> 1) ^ ((key >> 1) & 7u));
-  }
-  // B operand (dS^T, keys x heads) of head tile j: head row 16j + gi, keys 8g .. 8g+7
-  const uint32_t ds_lane = gi * 64u + 16u * (g ^ ((gi >> 1) & 3));
-  const int d0 = __builtin_amdgcn_readfirstlane(wave) * DT;   // first dim tile of this wave
-  const uint32_t tile0 = lds_addr(sm.ring.tile[0]);
-
-  // dQ^T accumulators: DT x HT tiles of 16 x 16, 288 registers per lane -- more than either
-  // register file: tiles 0..63 (row-major) are pinned in AccVGPRs, the rest in VGPRs
-  // (AGPR/VGPR-constrained MFMAs; left to itself the compiler moves tiles between the files
-  // around the MFMAs).
-  constexpr int kTilesA = 64;
-  f32x4 acc[DT][HT];
-#pragma unroll
-  for (int i = 0; i < DT; ++i)
-#pragma unroll
-    for (int j = 0; j < HT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  mfma_acc_drain();   // zero writes of the accumulators before their first MFMA read
-
-  if (nblk > 0) {
-    gather_tile<NW, ROPE>(tile0, p.kv, sm.idx, wave, lane);
-    copy_ds(sm.ring.ds[0], 0);
-  }
-  if (nblk > 1) {
-    gather_tile<NW, ROPE>(tile0 + kTileBytes, p.kv, sm.idx + kBK, wave, lane);
-    copy_ds(sm.ring.ds[1], 1);
-  }
-  int st = 0;   // ring stage of block blk
-  for (int blk = 0; blk < nblk; ++blk) {
-    if (blk + 1 < nblk) wait_vmcnt<G>(); else wait_vmcnt<0>();
-    __syncthreads();
-    // block blk+2's copies, one tile copy per dim step below, the dS copies at steps 1 and 3
-    const bool copy_next = blk + 2 < nblk;
-    const int st_next = st == 0 ? 2 : st - 1;   // (blk + 2) % 3
-    TileSrc<NW> next_src;
-    if (copy_next) next_src = tile_sources<NW, ROPE>(p.kv, sm.idx + (blk + 2) * kBK, wave, lane);
-    // source row of the next tile copy, read one copy slot ahead of its issue
-    const char* next_row = copy_next ? gather_row<NW>(next_src, 0) : nullptr;
-    __builtin_amdgcn_sched_barrier(0);
-    const uint32_t next_tile = tile0 + st_next * kTileBytes;
-    char* const next_ds = sm.ring.ds[st_next];
-    const uint32_t tb = tile0 + st * kTileBytes;   // 128-byte aligned: the rope XOR stays in its row
-    const char* dsl = sm.ring.ds[st] + ds_lane;
-    st = st == 2 ? 0 : st + 1;
-    uint32_t v0 = tb + kv[0], v1 = tb + kv[1], r0 = tb + kr[0], r1 = tb + kr[1];
-    asm volatile("" : "+v"(v0), "+v"(v1), "+v"(r0), "+v"(r1));
-    u32x4 b[HT];
-#pragma unroll
-    for (int j = 0; j < HT; ++j) b[j] = lds_load16(dsl + 1024 * j);
-    auto ld = [&](int i) {
-      const int D = d0 + i;   // wave-uniform
-      const uint32_t x0 = D < 32 ? v0 + 32u * D : r0 ^ (32u * (D - 32));
-      const uint32_t x1 = D < 32 ? v1 + 32u * D : r1 ^ (32u * (D - 32));
-      const u32x2 lo = lds_read_tr16(lds_ptr(x0)), hi = lds_read_tr16(lds_ptr(x1));
-      return u32x4{lo[0], lo[1], hi[0], hi[1]};
-    };
-    u32x4 a[kPre];
-#pragma unroll
-    for (int i = 0; i < kPre; ++i) a[i] = ld(i);
-#pragma unroll
-    for (int i = 0; i < DT; ++i) {
-      const u32x4 cur = a[i % kPre];
-      if (i + kPre < DT) a[i % kPre] = ld(i + kPre);
-#pragma unroll
-      for (int j = 0; j < HT; ++j) {
-        if (i * HT + j < kTilesA) mfma16x16x32_cA(acc[i][j], cur, b[j]);
-        else mfma16x16x32_cV(acc[i][j], cur, b[j]);
-      }
-      if (copy_next) {
-        if (i < TC) {
-          gather_issue<NW>(next_tile, next_src, next_row, wave, lane, i);
-          next_row = gather_row<NW>(next_src, i + 1);
-        }
-        if (i == 1 || i == 3) copy_ds_part(next_ds, blk + 2, i >> 1);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-  mfma_acc_drain();
-  // ---- epilogue: dQ rows through LDS (64 heads at a time), then coalesced 16-byte stores.
-  // Lane holds head 16j + gi, dims 16(d0 + i) + 4g .. +3 of tile (i, j).
-  bf16_t* dq_t = p.dq + (int64_t)t * p.dq_stride_t;
-#pragma unroll
-  for (int half = 0; half < (HT + 3) / 4; ++half) {
-    __syncthreads();   // ring (or the previous half) no longer read
-#pragma unroll
-    for (int j = 4 * half; j < HT && j < 4 * half + 4; ++j) {
-      char* row = sm.out[16 * (j - 4 * half) + gi];
-#pragma unroll
-      for (int i = 0; i < DT; ++i)
-        *reinterpret_cast<u32x2*>(row + 2 * (16 * (d0 + i) + 4 * g)) =
-            u32x2{pack_bf16x2(acc[i][j][0], acc[i][j][1]), pack_bf16x2(acc[i][j][2], acc[i][j][3])};
-    }
-    __syncthreads();
-    const int rows = min(64, hrows - 64 * half);
-    const int qc = (p.q_dim != kDv ? kDqk : kDv) / 8;   // 16-byte chunks of a dq row (512: no rope part)
-    for (int c = threadIdx.x; c < rows * qc; c += NW * 64) {
-      const int r = c / qc, q = c - r * qc;
-      *reinterpret_cast<u32x4*>(dq_t + (int64_t)(h0 + 64 * half + r) * (8 * qc) + 8 * q) =
-          lds_load16(sm.out[r] + 16 * q);
-    }
-  }
-}
-
-// B2 for 64 < n_heads <= 128: 8 waves, two per SIMD.  Waves 0-3 issue the block gathers (the
+// 8 waves, two per SIMD.  Waves 0-3 issue the block gathers (the
 // 4-wave copy split of the KV and dS tiles) and own 5 dim tiles each (dims 80w ..), waves 4-7
 // own 4 dim tiles each and only multiply, so a copy-issuing wave stalled on its copies leaves
 // its SIMD to its partner (with one wave per SIMD those stalls cost ~30% of the block).  Every
@@ -485,7 +332,11 @@ __global__ __launch_bounds__(512, 1) void bwd_dq8_kernel(SparseBwdParams p) {
     const int hs = h < hrows ? h : 0;
     async_copy16_nt(ds_base + blk * ds_blk + hs * (kBK * 2) + q * 16, base + i * 1024u);
   };
-  // operand addresses as in bwd_dq_kernel
+  // A operand (K^T, dims x keys) of dim tile D: lane (g, gi) gets dim 16D + gi, keys 8g .. 8g+7
+  // as two transposing reads of 4 keys (rows 8g + gi/4 and 8g + 4 + gi/4, 4 dims from
+  // 16D + 4(gi%4)).  V dims (D < 32): tile row key_row(key) (keys 8g + j sit 2 rows apart:
+  // conflict-free), byte kv[h] + 32D; rope dims: kr[h] ^ (32(D - 32)).  B operand (dS^T, keys x
+  // heads) of head tile j: head row 16j + gi, keys 8g .. 8g+7.
   uint32_t kv[2], kr[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -996,47 +847,39 @@ int launch_sparse_mla_bwd(const SparseBwdParams& p, hipStream_t stream, hipEvent
     if (ev && hipEventRecord(ev[i], stream) != hipSuccess) marks_ok = false;
   };
   mark(0);
-  const int nw = p.n_heads > 64 ? 4 : (p.n_heads > 32 ? 2 : 1);
-  const dim3 grid(xcd_grid(p.total_q, p.n_xcd), (p.n_heads + 127) / 128);
   // B4 first: it only depends on idx.
   launch_pair_csr(p.idx, p.idx_stride, p.total_q, p.topk, p.n_kv, p.causal, p.q_offset, p.csr_counts,
                   p.csr_offsets, p.pair_pos, stream);
   mark(1);
-  // B1, B2: 512-wide q rows (no rope part) take the instantiations without the rope k-steps
-  auto launch_sp_dq = [&](auto rope_c) {
-    constexpr bool R = decltype(rope_c)::value;
-    if (nw == 4) {
-      hipLaunchKernelGGL((bwd_sp_kernel<4, R>), grid, dim3(256), 0, stream, p);
-      mark(2);
-      if (grid.y == 1) hipLaunchKernelGGL((bwd_dq8_kernel<R>), grid, dim3(512), 0, stream, p);
-      else hipLaunchKernelGGL((bwd_dq_kernel<4, R>), grid, dim3(256), 0, stream, p);
-    } else if (nw == 2) {
-      hipLaunchKernelGGL((bwd_sp_kernel<2, R>), grid, dim3(128), 0, stream, p);
-      mark(2);
-      hipLaunchKernelGGL((bwd_dq_kernel<2, R>), grid, dim3(128), 0, stream, p);
-    } else {
-      hipLaunchKernelGGL((bwd_sp_kernel<1, R>), grid, dim3(64), 0, stream, p);
-      mark(2);
-      hipLaunchKernelGGL((bwd_dq_kernel<1, R>), grid, dim3(64), 0, stream, p);
-    }
-  };
-  if (p.q_dim == kDv) launch_sp_dq(std::false_type{});
-  else launch_sp_dq(std::true_type{});
+  // B1, B2: 512-wide q rows (no rope part) take the instantiations without the rope k-steps; up to
+  // 64 heads one kernel does both (11.3 M pairs of 16 heads 6.53 -> 1.21 ms, 3.15 M pairs of 64 heads 1.81 -> 1.50)
+  const dim3 grid(xcd_grid(p.total_q, p.n_xcd));
+  if (p.n_heads <= 64) {
+    launch_bwd_spdq_fh(p, stream);
+    mark(2);
+  } else if (p.q_dim == kDv) {
+    hipLaunchKernelGGL((bwd_sp_kernel<4, false>), grid, dim3(256), 0, stream, p);
+    mark(2);
+    hipLaunchKernelGGL((bwd_dq8_kernel<false>), grid, dim3(512), 0, stream, p);
+  } else {
+    hipLaunchKernelGGL((bwd_sp_kernel<4, true>), grid, dim3(256), 0, stream, p);
+    mark(2);
+    hipLaunchKernelGGL((bwd_dq8_kernel<true>), grid, dim3(512), 0, stream, p);
+  }
   mark(3);
   const int nks = p.n_heads / 16;
-  const dim3 ggrid(xcd_grid(p.total_q, p.n_xcd));
   // bf16 G rows of 512-wide q rows are 1024 bytes (no rope part); int8 rows keep their format
   const bool g512 = !p.g_int8 && p.q_dim == kDv;
   auto launch_g = [&](auto rope_c) {
     constexpr bool R = decltype(rope_c)::value;
     if (nks > 4)
-      hipLaunchKernelGGL((bwd_g_kernel<8, false, R>), ggrid, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((bwd_g_kernel<8, false, R>), grid, dim3(256), 0, stream, p);
     else if (nks > 2)
-      hipLaunchKernelGGL((bwd_g_kernel<4, false, R>), ggrid, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((bwd_g_kernel<4, false, R>), grid, dim3(256), 0, stream, p);
     else if (nks > 1)
-      hipLaunchKernelGGL((bwd_g_kernel<2, false, R>), ggrid, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((bwd_g_kernel<2, false, R>), grid, dim3(256), 0, stream, p);
     else
-      hipLaunchKernelGGL((bwd_g_kernel<1, false, R>), ggrid, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((bwd_g_kernel<1, false, R>), grid, dim3(256), 0, stream, p);
   };
   if (p.g_int8) launch_bwd_g_i8(p, stream);
   else if (g512) launch_g(std::false_type{});

@@ -23,9 +23,7 @@
 // through registers in the MFMA operand layout (1.86; its 64-byte pieces do not coalesce), the
 // k-split for two head tiles (1.43 against 1.28: a third barrier), four head tiles in one workgroup
 // per CU (2.73), the copies spread between the PV MFMAs (no change; spills at two head tiles).
-#include "dsa_common.h"
-#include "dsa_kernels.h"
-#include "dsa_kvtile.h"
+#include "dsa_fh.h"
 
 namespace dsa {
 
@@ -33,23 +31,7 @@ namespace {
 
 constexpr int kDqk = 576;
 constexpr int kDv = 512;
-constexpr int kBK = kTileKeys;
 constexpr float kHeadroom = 64.0f;      // log2 headroom above the reference max
-constexpr int kNW = 4;
-constexpr int kIdxSlots = 4;            // ring of index slices (block b's 32 entries at b % 4)
-
-// V row of block key k: keys 8j .. 8j+7 sit two rows apart, so that a transposing read of 32 lanes
-// (8 keys, 32 bytes each) covers all banks; 16 consecutive keys still cover 16 consecutive rows.
-constexpr uint32_t fh_row(uint32_t k) { return (k & 16u) | ((k & 7u) << 1) | ((k >> 3) & 1u); }
-
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-
-DSA_DEV u32x2 lds_read_tr16(const char* p) {
-  s16x4 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p));
-  return __builtin_bit_cast(u32x2, r);
-}
-
 template <int NHT>
 struct FhSmem {
   union {
@@ -57,9 +39,9 @@ struct FhSmem {
     char ostage[16 * NHT][kDv * 2];   // epilogue: bf16 output rows, chunk c of row r at c ^ (r & 7)
   };
   u32x4 xbuf[4][64];                  // NHT = 1: partial S^T of wave w; NHT = 2: P^T fragments of head tile n
-  int32_t idx[kIdxSlots][64];
+  int32_t idx[kFhIdxSlots][64];
   float m[16 * NHT], l[2][16 * NHT], seen[2][16 * NHT], inv_l[16 * NHT];
-  int red[kNW];
+  int red[kFhWaves];
 };
 
 }  // namespace
@@ -70,7 +52,6 @@ __global__ __launch_bounds__(256, 2) void sparse_mla_fwd_fh_kernel(SparseFwdPara
   constexpr int KS = NHT == 1 ? QKS / 2 : QKS;       // k-steps of a wave
   constexpr int KA = QKS / 2;                        // K fragments in registers
   constexpr int DT = 8;                              // 16-dim tiles of a wave's O^T
-  constexpr int G = tile_copies_per_wave<kNW, ROPE>();
   static_assert(sizeof(FhSmem<NHT>) <= 80 * 1024, "two workgroups per CU");
   __shared__ __attribute__((aligned(128))) FhSmem<NHT> sm;
 
@@ -100,31 +81,17 @@ __global__ __launch_bounds__(256, 2) void sparse_mla_fwd_fh_kernel(SparseFwdPara
       qf[i] = ok ? v : u32x4{0, 0, 0, 0};
     }
   }
-  // ---- last valid slot of the index row; the first blocks' slices
+  // ---- index row: blocks up to the last valid slot
   const int k_first = split * p.split_keys;
-  const int n_slots = max(0, min(p.topk - k_first, p.split_keys));
-  const int32_t* idx_row = p.idx + (int64_t)t * p.idx_stride + k_first;
-  const uint32_t lim = p.causal ? min(p.n_kv, t + 1) : p.n_kv;   // valid ids: 0 .. lim - 1
-  int last = -1;
-  {
-    constexpr int kBatch = 8;   // loads in flight per thread
-    for (int j0 = threadIdx.x; j0 < n_slots; j0 += kBatch * 256) {
-      int v[kBatch];
-#pragma unroll
-      for (int i = 0; i < kBatch; ++i) v[i] = j0 + i * 256 < n_slots ? idx_row[j0 + i * 256] : -1;
-#pragma unroll
-      for (int i = 0; i < kBatch; ++i)
-        if ((uint32_t)v[i] < lim) last = j0 + i * 256;
-      if (j0 < kIdxSlots * kBK) sm.idx[j0 / kBK][j0 % kBK] = v[0];
-    }
-  }
-  last = wave_max_i(last);
-  if (lane == 0) sm.red[wave] = last;
-  wait_vmcnt0();   // Q and index loads retired: nothing compiler-visible stays in flight
-  __syncthreads();
-#pragma unroll
-  for (int w = 0; w < kNW; ++w) last = max(last, sm.red[w]);
-  const int nblk = __builtin_amdgcn_readfirstlane((last + kBK) / kBK);
+  FhGather<ROPE> gth;
+  gth.kv = p.kv;
+  gth.idx_row = p.idx + (int64_t)t * p.idx_stride + k_first;
+  gth.slots = sm.idx;
+  gth.n_slots = max(0, min(p.topk - k_first, p.split_keys));
+  gth.lane = lane;
+  gth.wave = wave;
+  gth.lim = p.causal ? min(p.n_kv, t + 1) : p.n_kv;
+  const int nblk = gth.setup(sm.red);
 
   // score operand (A): key 16 kt + gi, chunk 4 ks + g.  NHT = 1, upper k half: the last two k-steps
   // lie in the rope region.
@@ -135,41 +102,6 @@ __global__ __launch_bounds__(256, 2) void sparse_mla_fwd_fh_kernel(SparseFwdPara
   const uint32_t pv_lo = fh_row(4 * g + (gi >> 2)) * kTileVPitch + 8u * (gi & 3) + 256u * wave;
   const uint32_t pv_hi = pv_lo + 16u * kTileVPitch;   // fh_row(k + 16) = fh_row(k) + 16
   const uint32_t tile0 = lds_addr(sm.tile[0]);
-
-  // a block's gather: sources from the raw entries of its index slice (rv: key wave + 4 (lane % 8),
-  // rr: key 8 wave + lane / 8; an invalid entry loads row 0), copies of keys wave + 4k and a rope
-  // group.  No branch between the reads of the entries and their use: a wait for one would be a
-  // wait for every LDS read in flight.
-  auto entry = [&](int blk, int key) { return (uint32_t)sm.idx[blk % kIdxSlots][key]; };
-  auto entry_ok = [&](uint32_t x, int blk, int key) { return (x < lim) & (blk * kBK + key < n_slots); };
-  const int key_v = wave + kNW * (lane & 7), key_r = 8 * wave + (lane >> 3);
-  auto sources = [&](int blk, uint32_t rv, uint32_t rr) {
-    TileSrc<kNW> src;
-    src.v = reinterpret_cast<const char*>(p.kv) + (uint64_t)(entry_ok(rv, blk, key_v) ? rv : 0u) * (kLatent * 2);
-    if constexpr (ROPE)
-      src.rope[0] = reinterpret_cast<const char*>(p.kv) + (uint64_t)(entry_ok(rr, blk, key_r) ? rr : 0u) * (kLatent * 2) +
-                    (64 + ((lane & 7) ^ ((key_r >> 1) & 7))) * 16;
-    return src;
-  };
-  auto gather = [&](uint32_t tile, const TileSrc<kNW>& src) {
-    const TileDst d = tile_dst<kNW>(tile, wave);   // row fh_row(wave) = 2 wave
-    const char* row[2] = {gather_row<kNW>(src, 0), gather_row<kNW>(src, 1)};
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_nop 4");
-    static_for<0, G>([&](auto kc) {
-      constexpr int k = decltype(kc)::value;
-      if constexpr (k < 8) copy_row16_at<fh_row(kNW * k) * kTileVPitch>(d.v, row[k & 1], (uint32_t)lane * 16u);
-      else copy16_at<0>(src.rope[0], d.rope);
-      row[k & 1] = gather_row<kNW>(src, k + 2);
-      __builtin_amdgcn_sched_barrier(0);
-    });
-  };
-  // index slice of block blk (past the row: its last entry again)
-  auto copy_idx = [&](int blk) {
-    if (wave == 0)
-      async_copy4_unordered(idx_row + min(blk * kBK + lane, n_slots - 1),
-                            __builtin_amdgcn_readfirstlane(lds_addr(sm.idx[blk % kIdxSlots])));
-  };
 
   auto max4 = [](const f32x4& x) { return fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])); };
   auto over_g = [](float v) {   // maximum over the four lane groups of a head
@@ -195,18 +127,10 @@ __global__ __launch_bounds__(256, 2) void sparse_mla_fwd_fh_kernel(SparseFwdPara
 #pragma unroll
       for (int n = 0; n < NHT; ++n) o[d][n] = f32x4{0.f, 0.f, 0.f, 0.f};
     l_run = 0.f;
-    if (pass == 1) {   // the slices have moved on: fetch the first ones again
-      for (int b = 0; b < kIdxSlots; ++b) copy_idx(b);
-      wait_vmcnt0();
-      __syncthreads();
-    }
-    // copies in flight behind a gather: wave 0 also copies a slice with each gather of the loop
-    for (int b = 0; b < min(nblk, 2); ++b) gather(tile0 + b * kTileBytes, sources(b, entry(b, key_v), entry(b, key_r)));
+    if (pass == 1) gth.restart();
+    gth.start(tile0, nblk);
     for (int blk = 0; blk < nblk; ++blk) {
-      // block blk's copies done; those of block blk + 1 (issued after them) may be in flight
-      if (blk + 1 >= nblk) wait_vmcnt0();
-      else if (blk > 0 && wave == 0) wait_vmcnt<G + 1>();
-      else wait_vmcnt<G>();
+      gth.template wait<0>(blk, nblk);
       __syncthreads();
       const uint32_t tb = tile0 + (blk & 1) * kTileBytes;
       uint32_t av = tb + s_v, ar = tb + s_r, lo = tb + pv_lo, hi = tb + pv_hi;
@@ -222,19 +146,20 @@ __global__ __launch_bounds__(256, 2) void sparse_mla_fwd_fh_kernel(SparseFwdPara
         }
         return lds_load16(lds_ptr(a));
       };
-      const uint32_t xm = entry(blk, lane & 31), xv = entry(blk + 2, key_v), xr = entry(blk + 2, key_r);
+      const uint32_t xm = gth.entry(blk, lane & 31);
+      const uint32_t xv = gth.entry(blk + 2, gth.key_v()), xr = gth.entry(blk + 2, gth.key_r());
       u32x4 ka[KA];
 #pragma unroll
       for (int i = 0; i < KA; ++i) ka[i] = k_read(i);
       u32x4 va[DT];
 #pragma unroll
       for (int d = 0; d < DT; ++d) {
-        const u32x2 a = lds_read_tr16(lds_ptr(lo + 32u * d)), b = lds_read_tr16(lds_ptr(hi + 32u * d));
+        const u32x2 a = fh_read_tr16(lo + 32u * d), b = fh_read_tr16(hi + 32u * d);
         va[d] = u32x4{a[0], a[1], b[0], b[1]};
       }
-      const uint32_t vmask = (uint32_t)__ballot(entry_ok(xm, blk, lane & 31));
+      const uint32_t vmask = (uint32_t)__ballot(gth.ok(xm, blk, lane & 31));
       const bool more = blk + 2 < nblk;
-      const TileSrc<kNW> src = sources(blk + 2, xv, xr);
+      const TileSrc<kFhWaves> src = gth.sources(blk + 2, xv, xr);
 
       // ---- S^T = K . Q^T
       f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -254,8 +179,8 @@ __global__ __launch_bounds__(256, 2) void sparse_mla_fwd_fh_kernel(SparseFwdPara
       };
       auto gather_next = [&]() {   // the tile is read by nobody any more
         if (more) {
-          copy_idx(blk + 4);
-          gather(tb, src);
+          gth.copy_slice(blk + 4);
+          gth.issue(tb, src);
         }
       };
       if constexpr (NHT == 1) {
@@ -364,7 +289,7 @@ __global__ __launch_bounds__(256, 2) void sparse_mla_fwd_fh_kernel(SparseFwdPara
   }
   __syncthreads();
   bf16_t* obase = p.out + (int64_t)item * p.out_stride_t + (int64_t)h0 * kDv;
-  for (int r = wave; r < min(16 * NHT, p.n_heads - h0); r += kNW)
+  for (int r = wave; r < min(16 * NHT, p.n_heads - h0); r += kFhWaves)
     *reinterpret_cast<u32x4*>(obase + (int64_t)r * kDv + 8 * lane) = lds_load16(sm.ostage[r] + 16 * (lane ^ (r & 7)));
 }
 
