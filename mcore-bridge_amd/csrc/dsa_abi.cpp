@@ -44,18 +44,59 @@ BwdLayout bwd_layout(int total_q, int n_kv, int n_heads, int topk, int flags = 0
   return L;
 }
 
+// The same backward with dKV by key tiles (dsa_sparse_bwd_dkv.hip) instead of per-pair rows: P and
+// scale * dS where bwd_layout has them, then the inverse index and the splits' partial tiles.
+struct DkvLayout {
+  size_t p_stage, ds_stage, inv, flags, used, part, total;
+};
+DkvLayout dkv_layout(int total_q, int n_kv, int n_heads, int topk) {
+  DkvLayout L{};
+  const size_t stage = align_up(sizeof(uint16_t) * (size_t)total_q * n_heads * topk_pad(topk));
+  const size_t tiles = dsa::dkv_tiles(n_kv), splits = dsa::dkv_splits(total_q, n_kv);
+  size_t off = 0;
+  L.p_stage = off; off += stage;
+  L.ds_stage = off; off += stage;
+  L.inv = off; off += align_up(sizeof(uint16_t) * tiles * total_q * dsa::kDkvKeys);
+  L.flags = off; off += align_up(tiles * total_q);
+  L.used = off; off += align_up(tiles * splits);
+  L.part = off; off += align_up(sizeof(float) * tiles * splits * dsa::kDkvKeys * kDqk);
+  L.total = off;
+  return L;
+}
 // Query rows per pass of the sparse backward for a workspace of `bytes`: total_q when the whole
 // layout fits, else the most whole units of kBwdChunkUnit rows whose layout fits (0: none).
+// bytes_of(rows) grows with the rows.
 constexpr int kBwdChunkUnit = 256;
-int bwd_chunk_rows(int total_q, int n_kv, int n_heads, int topk, size_t bytes, int flags) {
-  if (bwd_layout(total_q, n_kv, n_heads, topk, flags).total <= bytes) return total_q;
-  int lo = 0, hi = total_q / kBwdChunkUnit;   // units; layouts grow with the rows
+template <class F>
+int chunk_rows(int total_q, size_t bytes, F bytes_of) {
+  if (bytes_of(total_q) <= bytes) return total_q;
+  int lo = 0, hi = total_q / kBwdChunkUnit;   // units
   while (lo < hi) {
     const int mid = (lo + hi + 1) / 2;
-    if (bwd_layout(mid * kBwdChunkUnit, n_kv, n_heads, topk, flags).total <= bytes) lo = mid;
+    if (bytes_of(mid * kBwdChunkUnit) <= bytes) lo = mid;
     else hi = mid - 1;
   }
   return lo * kBwdChunkUnit;
+}
+
+// dKV by key tiles instead of per-pair rows?  The rows cost per selected pair, 0.53 ns at 16 heads as at
+// 128 (their bytes); the tiles per visible (query, key) pair and 16 heads, 0.044 ns (their matrix
+// work), with `visible` counted as if every query saw all keys the causal mask leaves it.  Whole
+// backward, rows / tiles in us (causal): T = 8192, K = 2048: 16 heads 8840 / 2839, 64 heads 12900 /
+// 10820, 128 heads 14950 / 18500; T = 4096, K = 512: 16 heads 1262 / 673, 64 heads 2058 / 2466;
+// T = 16384: 16 heads K = 2048 18150 / 8670, K = 512 5479 / 6046, 64 heads K = 2048 26300 / 31900.
+// The tiles take no int8 rows, and their scratch must not exceed the size the caller was told.
+constexpr double kRowsPerPair = 0.53, kTilesPerVisible = 0.044;   // ns
+bool dkv_by_tiles(int total_q, int n_kv, int n_heads, int topk, int flags, bool causal) {
+  if (flags != 0 || total_q >= (1 << 28) || topk >= 0xffff) return false;
+  // sum over the queries of min(limit, keys the query sees)
+  auto seen = [&](int limit) {
+    if (!causal) return (double)total_q * limit;
+    const double ramp = std::min(total_q, limit);   // queries that see fewer
+    return ramp * (ramp + 1) / 2 + (total_q - ramp) * limit;
+  };
+  if (seen(n_kv) * (n_heads / 16) * kTilesPerVisible > seen(std::min(topk, n_kv)) * kRowsPerPair) return false;
+  return dkv_layout(total_q, n_kv, n_heads, topk).total <= bwd_layout(total_q, n_kv, n_heads, topk).total;
 }
 
 struct IdxBwdLayout {
@@ -480,7 +521,12 @@ int sparse_bwd(const void* q, const void* kv, const int32_t* idx, const void* ou
     return DSA_ERR_INVALID_ARG;
   // query rows per pass: all of them when the whole layout fits the workspace, else the most
   // whole units of kBwdChunkUnit rows whose layout fits (the timed variant needs one pass)
-  const int chunk = bwd_chunk_rows(total_q, n_kv, n_heads, topk, workspace_bytes, flags);
+  int chunk = 0;
+  if (dkv_by_tiles(total_q, n_kv, n_heads, topk, flags, causal != 0))
+    chunk = chunk_rows(total_q, workspace_bytes, [&](int r) { return dkv_layout(r, n_kv, n_heads, topk).total; });
+  const bool tiles = chunk > 0;
+  if (!tiles)
+    chunk = chunk_rows(total_q, workspace_bytes, [&](int r) { return bwd_layout(r, n_kv, n_heads, topk, flags).total; });
   if (!workspace || chunk == 0 || !aligned16(workspace)) return DSA_ERR_WORKSPACE;
   if (stage_events && chunk < total_q) return DSA_ERR_WORKSPACE;
   DSA_CHECK_DEVICE(dev);
@@ -492,6 +538,17 @@ int sparse_bwd(const void* q, const void* kv, const int32_t* idx, const void* ou
   p.dkv = dkv;
   p.p_stage = reinterpret_cast<dsa::bf16_t*>(ws + L.p_stage);
   p.ds_stage = reinterpret_cast<dsa::bf16_t*>(ws + L.ds_stage);
+  dsa::DkvParams d{};
+  if (tiles) {   // (the pieces of L past P do not exist)
+    const DkvLayout D = dkv_layout(chunk, n_kv, n_heads, topk);
+    p.ds_stage = reinterpret_cast<dsa::bf16_t*>(ws + D.ds_stage);
+    d.inv = reinterpret_cast<uint16_t*>(ws + D.inv);
+    d.flags = reinterpret_cast<uint8_t*>(ws + D.flags);
+    d.used = reinterpret_cast<uint8_t*>(ws + D.used);
+    d.part = reinterpret_cast<float*>(ws + D.part);
+    d.n_tiles = dsa::dkv_tiles(n_kv);
+    d.n_split = dsa::dkv_splits(chunk, n_kv);
+  }
   p.g_stage = ws + L.g_stage;
   p.g_int8 = (flags & DSA_BWD_G_INT8) ? 1 : 0;
   p.pair_pos = reinterpret_cast<int64_t*>(ws + L.pair_pos);
@@ -523,7 +580,8 @@ int sparse_bwd(const void* q, const void* kv, const int32_t* idx, const void* ou
     p.dkv_accumulate = c0 > 0 ? 1 : 0;
     p.g_sink_row = (int64_t)rows * topk;
     p.delta_out = delta_out ? delta_out + (int64_t)c0 * n_heads : nullptr;
-    const int rc = dsa::launch_sparse_mla_bwd(p, as_stream(stream), reinterpret_cast<hipEvent_t const*>(stage_events));
+    const int rc = dsa::launch_sparse_mla_bwd(p, tiles ? &d : nullptr, as_stream(stream),
+                                              reinterpret_cast<hipEvent_t const*>(stage_events));
     if (rc != 0) return rc;
   }
   return DSA_OK;
@@ -651,8 +709,9 @@ int dsa_indexer_kl_target_from_bwd(const void* bwd_workspace, size_t bwd_workspa
   if (n_heads > 128 || n_heads % 16 != 0) return DSA_ERR_UNSUPPORTED;
   if (total_q == 0) return DSA_OK;
   if (!idx || !target) return DSA_ERR_INVALID_ARG;
-  const BwdLayout L = bwd_layout(total_q, n_kv, n_heads, topk);
-  if (!bwd_workspace || bwd_workspace_bytes < L.total || !aligned16(bwd_workspace)) return DSA_ERR_WORKSPACE;
+  const BwdLayout L = bwd_layout(total_q, n_kv, n_heads, topk);   // P at its head in either layout
+  if (!bwd_workspace || bwd_workspace_bytes < L.total || !aligned16(bwd_workspace))
+    return DSA_ERR_WORKSPACE;
   dsa::KlFromPParams p{};
   p.p_stage = reinterpret_cast<const dsa::bf16_t*>(static_cast<const char*>(bwd_workspace) + L.p_stage);
   p.idx = idx; p.target = target;

@@ -50,7 +50,7 @@ DSA_DEV u32x2 lds_read_tr16(const char* p) {
 // ------------------------------------------------------------------------------------------
 constexpr int kGHeads = 128;                        // B3 handles up to 128 heads (n_heads % 16 == 0)
 constexpr int kGKs = kGHeads / 16;                  // head k-steps
-constexpr int kStageTile = kGHeads * 64;            // one staged [128 heads][32 keys] bf16 tile
+constexpr int kStageTile = kGHeads * 64;            // one staged tile: 8 chunks [32 keys][16 heads] bf16
 constexpr int kQRound = 16 * kDqk * 2;              // Q bytes of one setup round (16 heads)
 constexpr int kORound = 16 * kDv * 2;               // dO bytes of one setup round
 constexpr int kRoundBytes = kQRound + kORound;
@@ -66,8 +66,8 @@ struct GSmem {
   union {
     char ring[kSetupStages][kRoundBytes];           // setup: Q / dO rows of 16 heads per round
     struct {
-      char st[kStages][2][kStageTile];              // [dS | P] tiles; 16-byte chunk c of head row h
-                                                    //   at chunk c ^ (2 * ((h >> 1) & 1))
+      char st[kStages][2][kStageTile];              // [dS | P] tiles: 1 KB chunks of 16 heads (units:
+                                                    //   stage_unit, dsa_common.h)
       union {
         char gtile[kBK * kGTilePitch];              // bf16 rows: fp32 G tile of the last finished
                                                     //   block; 16-byte chunk j of a row at
@@ -270,29 +270,26 @@ __global__ __launch_bounds__(256, 1) void bwd_g_kernel(SparseBwdParams p) {
     }
   }
 
-  // ---- key blocks: [dS | P] tiles (rows = heads, 32 keys each) through a 3-stage copy ring
-  // staged tiles of block b: [H heads][32 keys] bf16, contiguous (see B1)
+  // ---- key blocks: [dS | P] tiles through a 3-stage copy ring; staged tiles of block b: one 1 KB
+  // chunk per 16 heads, contiguous
   const char* dsb = reinterpret_cast<const char*>(p.ds_stage + (int64_t)t * p.n_heads * p.topk_pad);
   const char* psb = reinterpret_cast<const char*>(p.p_stage + (int64_t)t * p.n_heads * p.topk_pad);
   const int64_t st_blk = (int64_t)p.n_heads * kBK * 2;   // bytes per staged block tile
-  // copy c (0..3) of this wave's share of block blk's [dS | P] rows: rows 16*(w + (c/2)*NW) ..,
-  // dS for even c, P for odd c.  Head rows past n_heads re-read row 0 (valid memory; their
-  // k-steps multiply zeros).
+  // copy c (0..3) of this wave's share of block blk's [dS | P] chunks: head group w + (c/2)*NW, dS for
+  // even c, P for odd c.  Groups past n_heads re-read group 0 (valid memory; their k-steps
+  // multiply zeros).
   auto stage_part = [&](int s, int blk, int c) {
     const uint32_t b = __builtin_amdgcn_readfirstlane(lds_addr(sm.loop.st[s][c & 1]));
     const int i = wu + (c >> 1) * NW;
-    const int h = 16 * i + (lane >> 2);
-    const int hs = h < p.n_heads ? h : 0;
-    const int chunk = (lane & 3) ^ (2 * ((h >> 1) & 1));   // LDS chunk lane&3 <- global chunk
-    const int64_t off = blk * st_blk + hs * (kBK * 2) + chunk * 16;
-    async_copy16_nt(((c & 1) ? psb : dsb) + off, b + i * 1024u);
+    const int64_t off = blk * st_blk + (i < nks ? i : 0) * kStageChunk + stage_unit_src(lane);
+    async_copy16_nt(((c & 1) ? psb : dsb) + off, b + i * (uint32_t)kStageChunk);
   };
   auto stage = [&](int s, int blk) {
 #pragma unroll
     for (int c = 0; c < G; ++c) stage_part(s, blk, c);
   };
-  // B operand address of this lane inside a tile: head row 16*ks + tr_h, bytes 2*tr_c .. +8
-  const uint32_t b_off = tr_h * 64 + 16 * (((2 * tr_c) >> 4) ^ (2 * ((tr_h >> 1) & 1))) + ((2 * tr_c) & 15);
+  // B operand address of this lane inside a chunk: key lane % 32, heads 8 * hb .. +7
+  const uint32_t b_off = 16 * stage_unit(lane & 31, hb);
   // G tile row of this lane's accumulators: key lane % 32.  Chunk 8*qtile + 2*q4 + hb of tile
   // 4w + i sits at slot (8*(4w + i) + 2*q4) + (hb ^ (i & 1)), of the rope tile 16 + w at
   // (8*(16 + w) + 2*q4) + (hb ^ (w & 1)): per-lane bases plus immediates.
@@ -366,10 +363,8 @@ __global__ __launch_bounds__(256, 1) void bwd_g_kernel(SparseBwdParams p) {
 #pragma unroll
       for (int i = 0; i < NQ; ++i) acc[i] = f32x16{};
       auto load_b = [&](int ks, u32x4& bs, u32x4& bp) {
-        const u32x2 s_lo = lds_read_tr16(sd + ks * 1024), s_hi = lds_read_tr16(sd + ks * 1024 + 4 * 64);
-        const u32x2 p_lo = lds_read_tr16(sp + ks * 1024), p_hi = lds_read_tr16(sp + ks * 1024 + 4 * 64);
-        bs = u32x4{s_lo[0], s_lo[1], s_hi[0], s_hi[1]};
-        bp = u32x4{p_lo[0], p_lo[1], p_hi[0], p_hi[1]};
+        bs = lds_load16(sd + ks * kStageChunk);
+        bp = lds_load16(sp + ks * kStageChunk);
       };
       u32x4 bs, bp;
       load_b(0, bs, bp);
@@ -484,10 +479,8 @@ __global__ __launch_bounds__(256, 1) void bwd_g_kernel(SparseBwdParams p) {
       const char* sp = sm.loop.st[blk % kStages][1] + b_off;
       u32x4 bs[KS], bp[KS];
       auto load_b = [&](int ks) {
-        const u32x2 s_lo = lds_read_tr16(sd + ks * 1024), s_hi = lds_read_tr16(sd + ks * 1024 + 4 * 64);
-        const u32x2 p_lo = lds_read_tr16(sp + ks * 1024), p_hi = lds_read_tr16(sp + ks * 1024 + 4 * 64);
-        bs[ks] = u32x4{s_lo[0], s_lo[1], s_hi[0], s_hi[1]};
-        bp[ks] = u32x4{p_lo[0], p_lo[1], p_hi[0], p_hi[1]};
+        bs[ks] = lds_load16(sd + ks * kStageChunk);
+        bp[ks] = lds_load16(sp + ks * kStageChunk);
       };
       load_b(0);
       if (KS > 1) load_b(1);

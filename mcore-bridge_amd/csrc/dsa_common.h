@@ -40,19 +40,13 @@ DSA_DEV f32x4 mfma16x16x32(const bf16x8& a, const bf16x8& b, const f32x4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// C += A * B with B and C in AccVGPRs.  gfx950 MFMAs read any operand from AccVGPRs, but the
+// MFMAs with operands pinned in AccVGPRs.  gfx950 MFMAs read any operand from AccVGPRs, but the
 // compiler only ever feeds A/B from VGPRs (spilled fragments then cost 4 v_accvgpr_read per
-// MFMA); these forms let a kernel keep a loop-invariant B operand set in AccVGPRs.  Hazards the
+// MFMA); these forms let a kernel keep a loop-invariant operand set in AccVGPRs.  Hazards the
 // compiler cannot see inside the asm are covered here and by the caller:
 //   - s_nop 1 before the MFMA: 2 wait states after a VALU write of A or an AccVGPR write of B/C;
 //   - the caller issues mfma_acc_drain() before any VALU reads C (8-pass XDL result: 11 wait
 //     states needed, 16 given).
-DSA_DEV void mfma32x32x16_acc_first(f32x16& c, const u32x4& a, const u32x4& b) {
-  asm("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "a"(b));
-}
-DSA_DEV void mfma32x32x16_acc(f32x16& c, const u32x4& a, const u32x4& b) {
-  asm("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "a"(b));
-}
 // C += A * B with C pinned in AccVGPRs ("a") or VGPRs ("v") and A, B in VGPRs -- for kernels
 // whose accumulators exceed 256 registers, where the compiler would shuttle tiles between the
 // two files around every MFMA.  Same hazard contract as above.
@@ -71,6 +65,13 @@ DSA_DEV void mfma16x16x32_cA(f32x4& c, const u32x4& a, const u32x4& b) {
 }
 DSA_DEV void mfma16x16x32_cV(f32x4& c, const u32x4& a, const u32x4& b) {
   asm("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+}
+// C += A * B with A and C in AccVGPRs and B in VGPRs (same hazard contract).
+DSA_DEV void mfma32x32x16_aA_first(f32x16& c, const u32x4& a, const u32x4& b) {
+  asm("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=a"(c) : "a"(a), "v"(b));
+}
+DSA_DEV void mfma32x32x16_aA(f32x16& c, const u32x4& a, const u32x4& b) {
+  asm("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "a"(a), "v"(b));
 }
 DSA_DEV void mfma_acc_drain() {
   __builtin_amdgcn_sched_barrier(0);
@@ -235,5 +236,16 @@ inline int xcd_grid(int n, int n_xcd) {
   const int full = n_xcd * kXcdChunk;
   return n >= full ? (n + full - 1) / full * full : (n + n_xcd - 1) / n_xcd * n_xcd;
 }
+
+// Staged P / scale * dS tiles of the sparse backward: one 1 KB chunk [32 keys][16 heads] bf16 per
+// (query, key block, group of 16 heads).  In LDS, 16-byte unit (key k, head half c) of a chunk sits at
+// stage_unit(k, c): 16 consecutive keys of one half lie on 16 different units modulo 16 (reads of 8
+// heads per key), and so do both halves of keys {0-3, 8-11} and {4-7, 12-15} (transposing reads).
+DSA_DEV uint32_t stage_unit(uint32_t k, uint32_t c) { return 2 * (k ^ ((k >> 1) & 4u)) + (c ^ ((k >> 3) & 1u)); }
+// Key and head half of unit `u` (the inverse), and its byte offset in the chunk in global memory.
+DSA_DEV uint32_t stage_unit_key(uint32_t u) { return (u >> 1) ^ ((u >> 2) & 4u); }
+DSA_DEV uint32_t stage_unit_half(uint32_t u) { return (u & 1u) ^ ((u >> 4) & 1u); }
+DSA_DEV uint32_t stage_unit_src(uint32_t u) { return 32 * stage_unit_key(u) + 16 * stage_unit_half(u); }
+constexpr int kStageChunk = 1024;   // bytes
 
 }  // namespace dsa

@@ -81,10 +81,11 @@ __global__ __launch_bounds__(256) void indexer_kl_kernel(KlLossParams p) {
 }
 
 // The same target from the P tiles the sparse MLA backward stages (B1 recomputes P = exp(scale *
-// S - lse) for every head and stores it in bf16, [t][block][head][32 keys]): target[t, j] = (1/H)
-// sum_h P[t, h, j], no S recompute.  One workgroup per query; thread (c, h0) reads 8 keys of
-// heads h0, h0 + 64 per block, summed over the wave's heads with lane shuffles and over the
-// waves through LDS.  Blocks past the query's last valid slot were not staged: their slots are 0.
+// S - lse) for every head and stores it in bf16 chunks of 32 keys x 16 heads): target[t, j] = (1/H)
+// sum_h P[t, h, j], no S recompute.  One workgroup per query; lane (key, head half) of wave w reads 8
+// heads of its key in every 4th head group, summed in the lane, with its neighbour (the other half)
+// and over the waves through LDS.  Blocks past the query's last valid slot were not staged: their
+// slots are 0.
 __global__ __launch_bounds__(256) void kl_target_from_p_kernel(KlFromPParams p) {
   __shared__ float part[4][32];
   __shared__ int red[4];
@@ -103,27 +104,18 @@ __global__ __launch_bounds__(256) void kl_target_from_p_kernel(KlFromPParams p) 
   const int nblk = (last + kBK) / kBK;
   float* out = p.target + (int64_t)t * p.target_stride;
   const float inv_h = 1.f / (float)p.n_heads;
-  const int c = threadIdx.x & 3, h0 = threadIdx.x >> 2;
-  const bf16_t* base = p.p_stage + (int64_t)t * (p.topk_pad / kBK) * p.n_heads * kBK;
+  const int n_hg = p.n_heads / 16;
+  const char* base = reinterpret_cast<const char*>(p.p_stage) + (int64_t)t * (p.topk_pad / kBK) * n_hg * kStageChunk;
   for (int b = 0; b < nblk; ++b) {
-    const bf16_t* tile = base + (int64_t)b * p.n_heads * kBK;
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int h = h0; h < p.n_heads; h += 64) {
-      const u32x4 v = gload16(tile + h * kBK + 8 * c);
+    const char* tile = base + (int64_t)b * n_hg * kStageChunk + 16 * lane;
+    float acc = 0.f;
+    for (int hg = wave; hg < n_hg; hg += 4) {
+      const u32x4 v = gload16(tile + hg * kStageChunk);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        acc[2 * e] += bf16_lo(v[e]);
-        acc[2 * e + 1] += bf16_hi(v[e]);
-      }
+      for (int e = 0; e < 4; ++e) acc += bf16_lo(v[e]) + bf16_hi(v[e]);
     }
-#pragma unroll
-    for (int o = 4; o < 64; o <<= 1)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) acc[e] += __shfl_xor(acc[e], o, 64);
-    if (lane < 4) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) part[wave][8 * lane + e] = acc[e];
-    }
+    acc += __shfl_xor(acc, 1, 64);
+    if ((lane & 1) == 0) part[wave][lane >> 1] = acc;
     __syncthreads();
     if (threadIdx.x < kBK && b * kBK + (int)threadIdx.x < p.topk) {
       const int k = threadIdx.x;

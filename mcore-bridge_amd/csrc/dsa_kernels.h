@@ -50,8 +50,8 @@ struct SparseBwdParams {
   bf16_t* dq;           // [total_q, n_heads, 576]
   float* dkv;           // [n_kv, 576] fp32 (fully written, no accumulation into old contents)
   // workspace (carved by the C-ABI from one caller buffer)
-  bf16_t* p_stage;      // [total_q, topk_pad/32, n_heads, 32]  P (one contiguous tile per key block)
-  bf16_t* ds_stage;     // [total_q, topk_pad/32, n_heads, 32]  scale * dS
+  bf16_t* p_stage;      // [total_q, topk_pad/32, n_heads/16, 32 keys, 16 heads]  P (chunks: dsa_common.h)
+  bf16_t* ds_stage;     // the same of scale * dS
   char* g_stage;        // [total_q * topk + 1] G rows (g_int8 ? kGRowBytesI8 : kGRowBytesBf16
                         // bytes each), key-major order
   int64_t g_sink_row;   // last row of g_stage: write target of pairs that select nothing
@@ -67,6 +67,17 @@ struct SparseBwdParams {
   int n_xcd;            // XCDs of the device (xcd_remap / xcd_grid)
   int q_dim;            // 576, or 512 (q and dq rows without the rope part: it counts as zero)
   float* delta_out;     // [total_q, n_heads] rowsum(dO * O) written by B1 (token stride n_heads), or null
+};
+
+// dKV by key tiles (dsa_sparse_bwd_dkv.hip): its scratch, carved from the backward's workspace.
+constexpr int kDkvKeys = 128;      // keys per tile
+constexpr int kDkvQChunk = 16;     // consecutive queries of a split
+struct DkvParams {
+  uint16_t* inv;        // [n_tiles, total_q, 128] slot of each key in the query's index row, 0xffff = none
+  uint8_t* flags;       // [n_tiles, total_q] key subtiles the query selects from (bits 0-3), repeats (bit 7)
+  uint8_t* used;        // [n_tiles, n_split] 1: the split's partial is written, 2: a row repeats a key
+  float* part;          // [n_tiles, n_split, 128, 576]
+  int n_tiles, n_split;
 };
 
 struct IndexerParams {
@@ -235,7 +246,13 @@ int launch_sparse_mla_fwd(const SparseFwdParams& p, hipStream_t stream);
 // n_heads <= 64 (dsa_sparse_fwd_fh.hip); called by launch_sparse_mla_fwd
 int launch_sparse_mla_fwd_fh(const SparseFwdParams& p, hipStream_t stream);
 // ev (nullable): 6 events recorded around the stages B4 | B1 | B2 | B3 | B5.
-int launch_sparse_mla_bwd(const SparseBwdParams& p, hipStream_t stream, hipEvent_t const* ev);
+// d: null for per-pair rows (B3 .. B5), else dKV by key tiles (one pass over all queries)
+int launch_sparse_mla_bwd(const SparseBwdParams& p, const DkvParams* d, hipStream_t stream, hipEvent_t const* ev);
+int dkv_tiles(int n_kv);
+int dkv_splits(int total_q, int n_kv);
+void launch_dkv_inverse(const SparseBwdParams& p, const DkvParams& d, hipStream_t stream);
+void launch_dkv_tiles(const SparseBwdParams& p, const DkvParams& d, hipStream_t stream);
+void launch_dkv_sum(const SparseBwdParams& p, const DkvParams& d, hipStream_t stream);
 // B1 and B2 in one kernel for n_heads <= 64 (dsa_sparse_bwd_fh.hip), launched by
 // launch_sparse_mla_bwd.
 void launch_bwd_spdq_fh(const SparseBwdParams& p, hipStream_t stream);

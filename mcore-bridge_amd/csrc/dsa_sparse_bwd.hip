@@ -15,7 +15,7 @@
 // ~50 ms at S = 16k, so the scatter is done as bf16 partial rows grouped by key and reduced in a
 // streaming pass instead.
 //   B1 bwd_sp_kernel   per query: recompute S, P, dP (shared K/V operand reads), Delta fused;
-//                      stage P and scale*dS (bf16, [t][h][j]).
+//                      stage P and scale*dS (bf16 chunks of 32 keys x 16 heads, dsa_common.h).
 //   B2 bwd_dq_kernel   per query: dQ^T += K^T . dS^T over the gathered rows (K^T via transposing
 //                      LDS reads, dS^T tile copied into LDS next to the KV tile).
 //   B3 bwd_g_kernel    per query: G^T[576 x keys] = Q^T . dS + dO^T . P contracted over all
@@ -48,11 +48,11 @@ namespace dsa {
 
 namespace {
 
-// lo = keys k .. k+3 and hi = keys k+8 .. k+11 in the lower half-wave (lane l < 32), keys
-// k+4 .. k+7 and k+12 .. k+15 in the upper half (lane l + 32, same head).  One
+// lo = heads h .. h+3 and hi = heads h+8 .. h+11 in the lower half-wave (lane l < 32), heads
+// h+4 .. h+7 and h+12 .. h+15 in the upper half (lane l + 32, same key).  One
 // v_permlane32_swap per dword trades the lower half's hi for the upper half's lo, after which
-// the lower lane holds keys k .. k+7 and the upper lane k+8 .. k+15: one 16-byte store each.
-DSA_DEV u32x4 swap_key_halves(u32x2 lo, u32x2 hi) {
+// the lower lane holds heads h .. h+7 and the upper lane h+8 .. h+15: one 16-byte store each.
+DSA_DEV u32x4 swap_head_halves(u32x2 lo, u32x2 hi) {
   u32x4 r;
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
@@ -76,7 +76,8 @@ struct SpSmem {
     char ostage[4][32][kDv * 2];   // setup: O rows of each wave's 32 heads (for Delta)
   };
   int32_t idx[kMaxTopkBwd];
-  float lse[4][64];                // setup: LSE of each lane's head
+  float lse[4][64];                // setup: LSE of each lane's head; then [w][h]: log2 LSE of the wave's
+                                   //   heads (+inf: no key) and, at 32 + h, scale * Delta
   int red[4];
 };
 
@@ -94,7 +95,6 @@ __global__ __launch_bounds__(NW * 64, 1) void bwd_sp_kernel(SparseBwdParams p) {
   const int hb = lane >> 5, hl = lane & 31;
   const int head = blockIdx.y * 128 + wave * 32 + hl;
   const bool head_ok = head < p.n_heads;
-  const bool wave_stores = blockIdx.y * 128 + wave * 32 < p.n_heads;  // wave-uniform
   const int hsafe = head_ok ? head : 0;
 
   static_assert(NW <= 4, "O staging holds 4 waves");
@@ -149,16 +149,15 @@ __global__ __launch_bounds__(NW * 64, 1) void bwd_sp_kernel(SparseBwdParams p) {
   }
   delta = xor32_sum(delta);
   if (p.delta_out != nullptr && head_ok && hb == 0) p.delta_out[(int64_t)t * p.n_heads + head] = delta;
-  const float delta_s = delta * p.scale;
   const float lse = head_ok ? sm.lse[wave][lane] : -INFINITY;
-  const float lse2 = lse * kLog2e;
-  const bool row_live = lse != -INFINITY;
   __syncthreads();   // O staging dead: the union now holds the KV tile ring
+  sm.lse[wave][lane] = hb == 0 ? (lse == -INFINITY ? INFINITY : lse * kLog2e) : delta * p.scale;   // own wave's rows
 
-  // staged tiles: element (t, head, slot 32*b + k) at ((t * NB + b) * H + head) * 32 + k
-  // (NB = topk_pad / 32): each block's [H heads x 32 keys] tile is contiguous; after the half
-  // swap (swap_key_halves) lane writes keys 16*pr + 8*hb .. +7 of each block, pr = 0, 1
-  const int64_t stage_off = ((int64_t)t * (p.topk_pad / kBK) * p.n_heads + hsafe) * kBK + hb * 8;
+  // staged chunks (dsa_common.h) of head groups 2 * wave + pr, pr = 0, 1: after the half swap
+  // (swap_head_halves) lane writes heads 8*hb .. +7 of key hl, 1 KB per store instruction
+  const int hg0 = blockIdx.y * 8 + 2 * wave, n_hg = p.n_heads / 16;
+  const int64_t stage_off = ((int64_t)t * (p.topk_pad / kBK) * n_hg + hg0) * (kStageChunk / 2) + hl * 16 + hb * 8;
+  const bool st_ok[2] = {hg0 < n_hg, hg0 + 1 < n_hg};   // wave-uniform
   const int64_t stage_blk = (int64_t)p.n_heads * kBK;   // elements per staged block tile
   bf16_t* ps_row = p.p_stage + stage_off;
   bf16_t* ds_row = p.ds_stage + stage_off;
@@ -179,13 +178,13 @@ __global__ __launch_bounds__(NW * 64, 1) void bwd_sp_kernel(SparseBwdParams p) {
     // block blk-2.
     if (blk == 0) {
       if (nblk > 1) wait_vmcnt<G>(); else wait_vmcnt<0>();
-    } else if (blk == 1 || !wave_stores) {
+    } else if (blk == 1 || !st_ok[1]) {   // (a wave with one head group issues half the stores)
       wait_vmcnt<G>();
     } else {
       wait_vmcnt<G + S>();
     }
     __syncthreads();
-    const bool store_prev = blk > 0 && head_ok;   // wave_stores => the wave issues all S stores
+    const bool store_prev[2] = {blk > 0 && st_ok[0], blk > 0 && st_ok[1]};
     const int64_t store_j = (blk - 1) * stage_blk;
     // block blk+2's gather, one copy per kCopyEvery S/dP steps below.  Issued every iteration:
     // the last two re-gather block nblk-1 into the ring slot no block reads any more (so no copy
@@ -193,6 +192,7 @@ __global__ __launch_bounds__(NW * 64, 1) void bwd_sp_kernel(SparseBwdParams p) {
     const TileSrc<NW> next_src = tile_sources<NW, ROPE>(p.kv, sm.idx + min(blk + 2, nblk - 1) * kBK, wave, lane);
     // source row of the next copy, read one copy slot ahead of its issue
     const char* next_row = gather_row<NW>(next_src, 0);
+    asm volatile("" : "+s"(next_row));   // read here, ahead of the copy (not sunk to it)
     __builtin_amdgcn_sched_barrier(0);
     const uint32_t next_tile = tile0 + st_next;
     const TileDst nd = tile_dst<NW>(next_tile, wsg);
@@ -203,8 +203,8 @@ __global__ __launch_bounds__(NW * 64, 1) void bwd_sp_kernel(SparseBwdParams p) {
     asm volatile("" : "+v"(qv), "+v"(qr));
     const uint32_t vmask = (uint32_t)__ballot(sm.idx[blk * kBK + (lane & 31)] >= 0);
 
-    // S^T = K . Q^T and dP^T = V . dO^T share the A operand (V = K[:, :512]); the dO^T
-    // fragments and the dP accumulator stay in AccVGPRs (Q + dO = 272 registers per lane).
+    // S = Q . K^T and dP = dO . V^T share the B operand (V = K[:, :512]); the dO fragments and the
+    // dP accumulator stay in AccVGPRs (Q + dO = 272 registers per lane).  Lane: key hl, 16 heads.
     f32x16 s = f32x16{}, dp;
     {
       auto addr = [&](int ks) { return lds_ptr(ks < 32 ? (qv + 32u * ks) : (qr ^ (32u * (ks - 32)))); };
@@ -215,57 +215,63 @@ __global__ __launch_bounds__(NW * 64, 1) void bwd_sp_kernel(SparseBwdParams p) {
       for (int ks = 0; ks < QKS; ++ks) {
         const u32x4 cur = a[ks % kPre];
         if (ks + kPre < QKS) a[ks % kPre] = lds_load16(addr(ks + kPre));
-        s = mfma32x32x16(as_bf16x8(cur), as_bf16x8(qf[ks]), s);
-        if (ks == 0) mfma32x32x16_acc_first(dp, cur, df[0]);
-        else if (ks < kDv / 16) mfma32x32x16_acc(dp, cur, df[ks]);
+        s = mfma32x32x16(as_bf16x8(qf[ks]), as_bf16x8(cur), s);
+        if (ks == 0) mfma32x32x16_aA_first(dp, df[0], cur);
+        else if (ks < kDv / 16) mfma32x32x16_aA(dp, df[ks], cur);
         if (ks % kCopyEvery == 0) {
           gather_issue_dst<NW>(nd, next_src, next_row, lane, ks / kCopyEvery);
           next_row = gather_row<NW>(next_src, ks / kCopyEvery + 1);
+          asm volatile("" : "+s"(next_row));   // read here: not sunk past the stores' branches to its copy
         }
-        if (ks % 8 == 1 && ks < 32 && store_prev) {
-          const int q = ks / 8;   // 0..3: P then dS of key half pr = q / 2
-          if (q & 1) *reinterpret_cast<u32x4*>(ds_row + store_j + 16 * (q >> 1)) = dw[q >> 1];
-          else *reinterpret_cast<u32x4*>(ps_row + store_j + 16 * (q >> 1)) = pw[q >> 1];
+        if (ks % 8 == 1 && ks < 32 && store_prev[ks / 16]) {
+          const int pr = ks / 16;   // P then dS of head group pr
+          const int64_t at = store_j + pr * (kStageChunk / 2);
+          if ((ks / 8) & 1) *reinterpret_cast<u32x4*>(ds_row + at) = dw[pr];
+          else *reinterpret_cast<u32x4*>(ps_row + at) = pw[pr];
         }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
     mfma_acc_drain();
-    // P = 2^(scale_log2 * s - lse2) and scale * dS = P * (scale * dP - scale * Delta); key of
-    // element i = (i/4)*8 + 4*hb + i%4.  Partial blocks / dead heads take the masked path.
-    float pv[16];
-    if (vmask == 0xffffffffu && __all(row_live)) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) pv[i] = fast_exp2(__builtin_fmaf(s[i], p.scale_log2, -lse2));
-    } else {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int key = (i >> 2) * 8 + hb * 4 + (i & 3);
-        const bool ok = row_live && ((vmask >> key) & 1u);
-        pv[i] = ok ? fast_exp2(__builtin_fmaf(s[i], p.scale_log2, -lse2)) : 0.f;
-      }
-    }
-    u32x2 pk[4], dk[4];   // keys 8*q4 + 4*hb .. +3
+    // P = 2^(scale_log2 * s - lse2) and scale * dS = P * (scale * dP - scale * Delta); head of element
+    // i = (i/4)*8 + 4*hb + i%4 (a head with no key: lse2 = +inf, P = 0)
+    u32x2 pk[4], dk[4];   // heads 8*q4 + 4*hb .. +3
 #pragma unroll
     for (int q4 = 0; q4 < 4; ++q4) {
-      float dv[4];
+      const f32x4 l2 = *reinterpret_cast<const f32x4*>(&sm.lse[wave][8 * q4 + 4 * hb]);
+      const f32x4 dl = *reinterpret_cast<const f32x4*>(&sm.lse[wave][32 + 8 * q4 + 4 * hb]);
+      float pv[4], dv[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) dv[e] = pv[4 * q4 + e] * __builtin_fmaf(dp[4 * q4 + e], p.scale, -delta_s);
-      pk[q4] = u32x2{pack_bf16x2(pv[4 * q4], pv[4 * q4 + 1]), pack_bf16x2(pv[4 * q4 + 2], pv[4 * q4 + 3])};
+      for (int e = 0; e < 4; ++e) {
+        pv[e] = fast_exp2(__builtin_fmaf(s[4 * q4 + e], p.scale_log2, -l2[e]));
+        dv[e] = pv[e] * __builtin_fmaf(dp[4 * q4 + e], p.scale, -dl[e]);
+      }
+      pk[q4] = u32x2{pack_bf16x2(pv[0], pv[1]), pack_bf16x2(pv[2], pv[3])};
       dk[q4] = u32x2{pack_bf16x2(dv[0], dv[1]), pack_bf16x2(dv[2], dv[3])};
     }
+    // slots that hold no key: zeros, whatever row 0 gave (masked after the packing: a branch while
+    // the AccVGPR accumulator is live lets the allocator copy it inside its wait states)
+    if (vmask != 0xffffffffu) {
+      const uint32_t m = (vmask >> hl) & 1u ? 0xffffffffu : 0u;
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        pk[q4] &= m;
+        dk[q4] &= m;
+      }
+    }
 #pragma unroll
     for (int pr = 0; pr < 2; ++pr) {
-      pw[pr] = swap_key_halves(pk[2 * pr], pk[2 * pr + 1]);
-      dw[pr] = swap_key_halves(dk[2 * pr], dk[2 * pr + 1]);
+      pw[pr] = swap_head_halves(pk[2 * pr], pk[2 * pr + 1]);
+      dw[pr] = swap_head_halves(dk[2 * pr], dk[2 * pr + 1]);
     }
   }
-  if (nblk > 0 && head_ok) {
-    const int64_t j = (nblk - 1) * stage_blk;
+  if (nblk > 0) {
 #pragma unroll
     for (int pr = 0; pr < 2; ++pr) {
-      *reinterpret_cast<u32x4*>(ps_row + j + 16 * pr) = pw[pr];
-      *reinterpret_cast<u32x4*>(ds_row + j + 16 * pr) = dw[pr];
+      if (!st_ok[pr]) continue;
+      const int64_t at = (nblk - 1) * stage_blk + pr * (kStageChunk / 2);
+      *reinterpret_cast<u32x4*>(ps_row + at) = pw[pr];
+      *reinterpret_cast<u32x4*>(ds_row + at) = dw[pr];
     }
   }
   wait_vmcnt0();   // the last re-gathers have landed in LDS before the workgroup ends
@@ -277,14 +283,14 @@ __global__ __launch_bounds__(NW * 64, 1) void bwd_sp_kernel(SparseBwdParams p) {
 // heads: K^T fragments (transposing reads of the KV tile) are read once per workgroup.  (Split by
 // heads instead, every wave would read the whole K^T tile for 36 MFMAs: four times the LDS reads.)
 // ------------------------------------------------------------------------------------------
-constexpr int kDsTileBytes = 128 * 64;  // [128 heads][32 keys] bf16
+constexpr int kDsTileBytes = 128 * 64;  // [8 head groups][32 keys][16 heads] bf16
 constexpr int kDqPitch = kDqk * 2 + 16;  // LDS pitch of a staged bf16 dQ row
 
 struct DqSmem {
   union {
     struct {
       char tile[kStages][kTileBytes];
-      char ds[kStages][kDsTileBytes];   // 16-byte chunk q of head row h at q ^ ((h >> 1) & 3)
+      char ds[kStages][kDsTileBytes];   // 1 KB chunk of head group i at i; units: stage_unit (dsa_common.h)
     } ring;
     char out[64][kDqPitch];             // epilogue: bf16 dQ rows of 64 heads
   };
@@ -320,23 +326,22 @@ __global__ __launch_bounds__(512, 1) void bwd_dq8_kernel(SparseBwdParams p) {
   const int nblk = stage_index_row<NW>(sm.idx, sm.red, p.idx + (int64_t)t * p.idx_stride, p.topk, p.n_kv,
                                        p.causal, t + p.q_offset);
   const int hrows = min(128, p.n_heads);
-  const char* ds_base = reinterpret_cast<const char*>(p.ds_stage + (int64_t)t * (p.topk_pad / kBK) * p.n_heads * kBK);
-  const int64_t ds_blk = (int64_t)p.n_heads * kBK * 2;   // bytes per staged block tile
-  // dS copy k (0, 1) of copy-issuing wave w: head rows 16 * (w + 4k) .. +15 (rows past n_heads
-  // re-read row 0; never stored)
+  const int n_hg = p.n_heads / 16;
+  const char* ds_base = reinterpret_cast<const char*>(p.ds_stage) + (int64_t)t * (p.topk_pad / kBK) * n_hg * kStageChunk;
+  const int64_t ds_blk = (int64_t)n_hg * kStageChunk;   // bytes per staged block
+  // dS copy k (0, 1) of copy-issuing wave w: head group w + 4k (groups past n_heads re-read group 0;
+  // never stored)
   auto copy_ds_part = [&](char* dst, int blk, int k) {
     const uint32_t base = __builtin_amdgcn_readfirstlane(lds_addr(dst));
     const int i = wu + k * NWC;
-    const int h = 16 * i + (lane >> 2);
-    const int q = (lane & 3) ^ ((h >> 1) & 3);
-    const int hs = h < hrows ? h : 0;
-    async_copy16_nt(ds_base + blk * ds_blk + hs * (kBK * 2) + q * 16, base + i * 1024u);
+    const int hg = i < n_hg ? i : 0;
+    async_copy16_nt(ds_base + blk * ds_blk + hg * kStageChunk + stage_unit_src(lane), base + i * (uint32_t)kStageChunk);
   };
   // A operand (K^T, dims x keys) of dim tile D: lane (g, gi) gets dim 16D + gi, keys 8g .. 8g+7
   // as two transposing reads of 4 keys (rows 8g + gi/4 and 8g + 4 + gi/4, 4 dims from
   // 16D + 4(gi%4)).  V dims (D < 32): tile row key_row(key) (keys 8g + j sit 2 rows apart:
   // conflict-free), byte kv[h] + 32D; rope dims: kr[h] ^ (32(D - 32)).  B operand (dS^T, keys x
-  // heads) of head tile j: head row 16j + gi, keys 8g .. 8g+7.
+  // heads) of head tile j: lane gets head 16j + gi, keys 8g .. 8g+7 as two transposing reads.
   uint32_t kv[2], kr[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -344,7 +349,10 @@ __global__ __launch_bounds__(512, 1) void bwd_dq8_kernel(SparseBwdParams p) {
     kv[h] = key_row(key) * kTileVPitch + 8u * (gi & 3);
     kr[h] = kTileVBytes + key * 128u + 8u * (gi & 1) + 16u * (((gi & 3) >> 1) ^ ((key >> 1) & 7u));
   }
-  const uint32_t ds_lane = gi * 64u + 16u * (g ^ ((gi >> 1) & 3));
+  uint32_t ds_lane[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    ds_lane[h] = 16u * stage_unit(8 * g + 4 * h + (gi >> 2), (gi & 3) >> 1) + 8u * (gi & 1);
   const int d0 = copier ? DTMAX * wu : DTMAX * NWC + DTP * (wu - NWC);   // first dim tile
   const int nd = copier ? DTMAX : DTP;
   const uint32_t tile0 = lds_addr(sm.ring.tile[0]);
@@ -390,7 +398,13 @@ __global__ __launch_bounds__(512, 1) void bwd_dq8_kernel(SparseBwdParams p) {
       const uint32_t next_tile = tile0 + st_next * kTileBytes;
       char* const next_ds = sm.ring.ds[st_next];
       const uint32_t tb = tile0 + st * kTileBytes;
-      const char* dsl = sm.ring.ds[st] + ds_lane;
+      const uint32_t dsl = lds_addr(sm.ring.ds[st]);
+      uint32_t b0 = dsl + ds_lane[0], b1 = dsl + ds_lane[1];
+      asm volatile("" : "+v"(b0), "+v"(b1));
+      auto ld_ds = [&](int j) {
+        const u32x2 lo = lds_read_tr16(lds_ptr(b0 + 1024u * j)), hi = lds_read_tr16(lds_ptr(b1 + 1024u * j));
+        return u32x4{lo[0], lo[1], hi[0], hi[1]};
+      };
       st = st == 2 ? 0 : st + 1;
       uint32_t v0 = tb + kv[0], v1 = tb + kv[1], r0 = tb + kr[0], r1 = tb + kr[1];
       asm volatile("" : "+v"(v0), "+v"(v1), "+v"(r0), "+v"(r1));
@@ -413,7 +427,7 @@ __global__ __launch_bounds__(512, 1) void bwd_dq8_kernel(SparseBwdParams p) {
       u32x4 a[ND];
 #pragma unroll
       for (int i = 0; i < ND; ++i) a[i] = ld(i);
-      u32x4 bq[2] = {lds_load16(dsl), lds_load16(dsl + 1024)};
+      u32x4 bq[2] = {ld_ds(0), ld_ds(1)};
 #pragma unroll
       for (int j = 0; j < HT; ++j) {
         const u32x4 bj = bq[j & 1];
@@ -427,7 +441,7 @@ __global__ __launch_bounds__(512, 1) void bwd_dq8_kernel(SparseBwdParams p) {
           }
         }
         copy_slot(2 * j + 1);
-        if (j + 2 < HT) bq[j & 1] = lds_load16(dsl + 1024 * (j + 2));
+        if (j + 2 < HT) bq[j & 1] = ld_ds(j + 2);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -838,18 +852,21 @@ void launch_pair_csr(const int32_t* idx, int64_t idx_stride, int total_q, int to
                      causal, t_offset, csr_offsets, csr_counts, pair_pos);
 }
 
-int launch_sparse_mla_bwd(const SparseBwdParams& p, hipStream_t stream, hipEvent_t const* ev) {
+int launch_sparse_mla_bwd(const SparseBwdParams& p, const DkvParams* d, hipStream_t stream, hipEvent_t const* ev) {
   if (p.n_xcd < 1) return -1;
   if (p.topk > kMaxTopkBwd) return -2;
-  if (p.g_sink_row >= INT32_MAX) return -2;   // B3 keeps G row numbers in 32 bits
+  if (!d && p.g_sink_row >= INT32_MAX) return -2;   // B3 keeps G row numbers in 32 bits
   bool marks_ok = true;   // a failed event record is reported like a failed launch
   auto mark = [&](int i) {
     if (ev && hipEventRecord(ev[i], stream) != hipSuccess) marks_ok = false;
   };
   mark(0);
-  // B4 first: it only depends on idx.
-  launch_pair_csr(p.idx, p.idx_stride, p.total_q, p.topk, p.n_kv, p.causal, p.q_offset, p.csr_counts,
-                  p.csr_offsets, p.pair_pos, stream);
+  // B4 (or the inverse index) first: it only depends on idx.
+  if (d)
+    launch_dkv_inverse(p, *d, stream);
+  else
+    launch_pair_csr(p.idx, p.idx_stride, p.total_q, p.topk, p.n_kv, p.causal, p.q_offset, p.csr_counts,
+                    p.csr_offsets, p.pair_pos, stream);
   mark(1);
   // B1, B2: 512-wide q rows (no rope part) take the instantiations without the rope k-steps; up to
   // 64 heads one kernel does both (11.3 M pairs of 16 heads 6.53 -> 1.21 ms, 3.15 M pairs of 64 heads 1.81 -> 1.50)
@@ -867,6 +884,13 @@ int launch_sparse_mla_bwd(const SparseBwdParams& p, hipStream_t stream, hipEvent
     hipLaunchKernelGGL((bwd_dq8_kernel<true>), grid, dim3(512), 0, stream, p);
   }
   mark(3);
+  if (d) {
+    launch_dkv_tiles(p, *d, stream);
+    mark(4);
+    launch_dkv_sum(p, *d, stream);
+    mark(5);
+    return hipGetLastError() == hipSuccess && marks_ok ? 0 : -4;
+  }
   const int nks = p.n_heads / 16;
   // bf16 G rows of 512-wide q rows are 1024 bytes (no rope part); int8 rows keep their format
   const bool g512 = !p.g_int8 && p.q_dim == kDv;

@@ -41,6 +41,32 @@ struct BwdFhSmem {
   int red[kFhWaves];
 };
 
+// 4 x 4 transpose of 16-bit values inside each quad of lanes: lane j of a quad holds elements
+// 0 .. 3 of row j and receives element j of rows 0 .. 3.
+struct QuadTranspose {
+  uint32_t keep, send, o0, o1;
+  bool upper;
+  DSA_DEV explicit QuadTranspose(int lane) {
+    // v_perm_b32(r, k, sel): bytes 0-3 of k, 4-7 of r
+    constexpr uint32_t lo = 0x05040100u, hi = 0x07060302u, lo_x = 0x01000504u, hi_x = 0x03020706u;
+    const int j = lane & 3;
+    upper = j & 2;
+    keep = (j & 1) ? hi : lo;
+    send = (j & 1) ? lo : hi;
+    o0 = j == 0 ? lo : j == 1 ? lo_x : j == 2 ? hi : hi_x;
+    o1 = j == 0 ? hi : j == 1 ? hi_x : j == 2 ? lo : lo_x;
+  }
+  DSA_DEV u32x2 operator()(const u32x2& x) const {
+    // elements {0, 1} or {2, 3} of rows j and j ^ 2, then the lane's element of all four rows
+    const uint32_t mine = upper ? x[1] : x[0], theirs = upper ? x[0] : x[1];
+    const uint32_t pair = __builtin_amdgcn_update_dpp(0, theirs, 0x4E, 0xf, 0xf, true);   // lane ^ 2
+    const uint32_t k = __builtin_amdgcn_perm(pair, mine, keep);      // rows j, j ^ 2
+    const uint32_t s = __builtin_amdgcn_perm(pair, mine, send);
+    const uint32_t r = __builtin_amdgcn_update_dpp(0, s, 0xB1, 0xf, 0xf, true);           // lane ^ 1: rows j ^ 1, j ^ 3
+    return u32x2{__builtin_amdgcn_perm(r, k, o0), __builtin_amdgcn_perm(r, k, o1)};
+  }
+};
+
 }  // namespace
 
 template <int NHT, bool ROPE>
@@ -120,10 +146,12 @@ __global__ __launch_bounds__(256, NHT == 1 ? 2 : 1) void bwd_spdq_fh_kernel(Spar
   const float delta_s = delta * p.scale, lse2 = lse * kLog2e;
   const bool live = lse != -INFINITY;
 
-  // staged tiles (dsa_sparse_bwd.hip): key slot 32 b + k of head h at ((t * NB + b) * H + h) * 32 + k;
-  // this lane: keys 16 kt + 4g .. +3 of its head.  NHT = 1: waves 0, 1 store P, waves 2, 3 dS.
-  const int64_t st0 = ((int64_t)t * (p.topk_pad / kBK) * p.n_heads + hs) * kBK + 16 * kt + 4 * g;
-  const int64_t st_blk = (int64_t)p.n_heads * kBK;
+  // staged chunks (dsa_common.h): after a 4 x 4 transpose in each lane quad, this lane holds key
+  // 16 kt + 4g + lane % 4 of four heads.  NHT = 1: waves 0, 1 store P, waves 2, 3 dS.
+  const int64_t st0 = ((int64_t)t * (p.topk_pad / kBK) * (p.n_heads / 16) + (hs >> 4)) * (kStageChunk / 2) +
+                      (16 * kt + 4 * g + (lane & 3)) * 16 + (gi & ~3);
+  const int64_t st_blk = (int64_t)p.n_heads * kBK;   // elements per block
+  const QuadTranspose quad(lane);
   bf16_t* const ps = p.p_stage + st0;
   bf16_t* const ds = p.ds_stage + st0;
 
@@ -225,7 +253,7 @@ __global__ __launch_bounds__(256, NHT == 1 ? 2 : 1) void bwd_spdq_fh_kernel(Spar
       const u32x2 x0 = pack4(dscore(pr[0], d[0])), x1 = pack4(dscore(pr[1], d[1]));
       bf[0] = u32x4{x0[0], x0[1], x1[0], x1[1]};
       bf16_t* const dst = (wr ? ds : ps) + blk * st_blk;
-      *reinterpret_cast<u32x2*>(dst) = wr ? (kt ? x1 : x0) : pack4(s);
+      *reinterpret_cast<u32x2*>(dst) = quad(wr ? (kt ? x1 : x0) : pack4(s));
     } else {
       const f32x4 pr = prob(s);
       const u32x2 x = pack4(dscore(pr, dp));
@@ -235,8 +263,8 @@ __global__ __launch_bounds__(256, NHT == 1 ? 2 : 1) void bwd_spdq_fh_kernel(Spar
       for (int n = 0; n < NHT; ++n) bf[n] = lds_load16(&sm.xbuf[n][lane]);
       refill();
       if (head_ok) {
-        *reinterpret_cast<u32x2*>(ps + blk * st_blk) = pack4(pr);
-        *reinterpret_cast<u32x2*>(ds + blk * st_blk) = x;
+        *reinterpret_cast<u32x2*>(ps + blk * st_blk) = quad(pack4(pr));
+        *reinterpret_cast<u32x2*>(ds + blk * st_blk) = quad(x);
       }
     }
     // ---- dQ^T += K^T . dS^T

@@ -173,7 +173,7 @@ def _violations(asm_text):
     return bad
 
 
-@pytest.mark.parametrize("src", ["dsa_sparse_fwd.hip", "dsa_sparse_fwd_fh.hip", "dsa_sparse_bwd.hip", "dsa_sparse_bwd_fh.hip", "dsa_indexer.hip", "dsa_indexer_bwd.hip",
+@pytest.mark.parametrize("src", ["dsa_sparse_fwd.hip", "dsa_sparse_fwd_fh.hip", "dsa_sparse_bwd.hip", "dsa_sparse_bwd_fh.hip", "dsa_sparse_bwd_dkv.hip", "dsa_indexer.hip", "dsa_indexer_bwd.hip",
                                  "dsa_dense_kl.hip"])
 def test_no_valu_write_right_before_mfma(src, tmp_path):
     out = tmp_path / (src + ".s")

@@ -108,3 +108,52 @@ def test_few_heads_backward(H, K):
             err = (got.double().cpu() - ref).norm().item()
             assert err < 1e-2 * ref.norm().item() + floor, f"{name} causal={causal}: {err} of {ref.norm()}"
         assert torch.equal(dkv, ops.sparse_mla_bwd(*a, SCALE, causal)[1])
+
+
+# (T, N, K, H, causal, q width): key tiles of 128 and subtiles of 32 that end inside, query chunks of 16,
+# two LDS passes of the inverse index (N > 16384), one to eight head groups; at each of them a query
+# selects a good part of the keys it sees, so dKV is summed by key tiles
+_TILED = [(130, 129, 96, 16, False, 576), (128, 128, 128, 48, True, 576), (257, 257, 200, 64, True, 576),
+          (513, 300, 256, 128, False, 576), (20, 16500, 1600, 16, False, 576), (145, 161, 160, 32, False, 512)]
+
+
+@pytest.mark.parametrize("T,N,K,H,causal,dqk", _TILED)
+def test_backward_by_key_tiles(T, N, K, H, causal, dqk):
+    from mcore_bridge_amd import ops
+    print(f"[key tiles] T={T} N={N} K={K} H={H} causal={causal} {dqk}", flush=True)
+    g = torch.Generator().manual_seed(T + N + H)
+    q = torch.randn(T, H, dqk, generator=g).bfloat16()
+    kv = torch.randn(N, 576, generator=g).bfloat16()
+    kv[:, dqk:] = 0
+    dout = torch.randn(T, H, 512, generator=g).bfloat16()
+    idx = _rows(T, N, K, T, causal)
+    idx[9, 4], idx[9, 7], idx[10, 1] = idx[9, 2], idx[9, 2], idx[10, 3]   # rows that repeat a key
+    ok = (idx >= 0) & (idx < N)
+    if causal:
+        ok &= idx <= torch.arange(T)[:, None]
+    ref_idx = torch.where(ok, idx, torch.full_like(idx, -1)).long()
+    qp = torch.nn.functional.pad(q, (0, 576 - dqk))
+    o_ref, l_ref = O.sparse_mla_fwd(qp, kv, ref_idx, SCALE)
+    out, lse = o_ref.bfloat16(), l_ref.float()
+    dq_ref, dkv_ref = O.sparse_mla_bwd(qp, kv, ref_idx, out, dout, l_ref, SCALE)
+    a = [x.to(DEV) for x in (q, kv, idx, out, dout, lse)]
+    far = torch.full((H,), -1e4, device=DEV)   # 512-wide rows come with a sink: one of no weight
+
+    def bwd(*cap):
+        return ops.sparse_mla_bwd(*a, SCALE, causal, *cap) if dqk == 576 else ops.sparse_mla_bwd_sink(*a, far, SCALE, causal)[:2]
+
+    dq, dkv = bwd()
+    assert _err(dq, dq_ref[..., :dqk]) < 1e-2 and _err(dkv, dkv_ref) < 1e-2
+    assert torch.equal(dkv, bwd()[1])
+    if T > 512:   # passes of 256 queries under a cap
+        one = ops.bwd_workspace_bytes_chunked(T, N, H, K, 256)
+        dq2, dkv2 = bwd(one)
+        assert torch.equal(dq2, dq) and _err(dkv2, dkv_ref) < 1e-2
+    # a query that is not finite reaches the keys it selects and no other
+    a[0][T - 2, H // 2, 3] = float("inf")
+    bad = torch.zeros(N, dtype=torch.bool)
+    bad[idx[T - 2][ok[T - 2]].long()] = True
+    dkv = bwd()[1].cpu()
+    assert torch.equal(~torch.isfinite(dkv).all(1), bad)
+    rest = O.sparse_mla_bwd(qp, kv, torch.where(torch.arange(T)[:, None] == T - 2, -1, ref_idx), out, dout, l_ref, SCALE)[1]
+    assert _err(dkv[~bad], rest[~bad]) < 1e-2
