@@ -34,7 +34,7 @@
 // stable compaction pass (each wave ranks 64 consecutive keys per step with ballots) then emits
 // every larger key plus the lowest-index ties.  Every path emits the same indices: ascending key
 // order, -1 padded.  Fewer than 256 rows longer than a slice (decode) are split: a workgroup
-// per (row, 16384-key slice) keeps the slice's top-K, one per row then selects from those.
+// per (row, 65536-key slice) keeps the slice's top-K, one per row then selects from those.
 #include <algorithm>
 #include "dsa_common.h"
 #include "dsa_kernels.h"
@@ -917,26 +917,21 @@ DSA_DEV int block_excl_scan(int v, int* sh, int* total) {
   return before + incl - v;
 }
 
-// True when key u lies under `prefix` in the bits at and above hi_shift (all keys when hi_shift = 32).
-DSA_DEV bool under_prefix(uint32_t u, uint32_t prefix, int hi_shift) {
-  return hi_shift >= 32 || (u >> hi_shift) == (prefix >> hi_shift);
-}
-
-// One histogram window of a radix select over the m keys in LDS that lie under `prefix` above
-// hi_shift: bins (u >> shift) & (nb - 1), nb = 2^(hi_shift - shift) <= 2048 (hist: 2048 ints).
-// Returns the bin holding the need-th largest of those keys (need >= 1 of them exist), with
-// *above = their keys in higher bins and *in_bin = the bin's keys.  sel: 3 ints, written by one
-// thread between two barriers and read after the second; the caller passes a barrier before
-// sel[0..2], hist or sh is written again.
-DSA_DEV int window_pass(const uint32_t* keys, int m, uint32_t prefix, int hi_shift, int shift, int need, int* hist,
+// One histogram window over those of the m keys in LDS that lie in [lo, lo + last]: bins
+// (u - lo) >> shift, at most 2048 (hist: 2048 ints).  Returns the bin holding the need-th largest of
+// those keys (need >= 1 of them exist), with *above = their keys in higher bins and *in_bin = the
+// bin's keys.  sel: 3 ints, written by one thread between two barriers and read after the second; the
+// caller passes a barrier before sel[0..2], hist or sh is written again.
+DSA_DEV int window_shift(uint32_t last) { return max(0, 21 - __clz(last)); }   // last >> shift < 2048
+DSA_DEV int window_pass(const uint32_t* keys, int m, uint32_t lo, uint32_t last, int shift, int need, int* hist,
                         int* sh, int* sel, int* above, int* in_bin) {
   constexpr int T = kTopkThreads;
-  const int nb = 1 << (hi_shift - shift);
+  const int nb = (int)(last >> shift) + 1;
   for (int b = threadIdx.x; b < nb; b += T) hist[b] = 0;
   __syncthreads();
   for (int i = threadIdx.x; i < m; i += T) {
-    const uint32_t u = keys[i];
-    if (under_prefix(u, prefix, hi_shift)) atomicAdd(&hist[(u >> shift) & (uint32_t)(nb - 1)], 1);
+    const uint32_t d = keys[i] - lo;
+    if (d <= last) atomicAdd(&hist[d >> shift], 1);
   }
   __syncthreads();
   // bins in descending order, 4 per thread: thread t holds bins nb-1-4t .. nb-4-4t
@@ -969,28 +964,26 @@ DSA_DEV int window_pass(const uint32_t* keys, int m, uint32_t prefix, int hi_shi
 }
 
 // Exact need-th largest of the m keys in LDS (lo <= every key <= hi, need <= m): thr, and how
-// many of the keys equal to it fall within the need largest.  Histogram windows of up to 11
-// bits below the common prefix of lo and hi; once the chosen bin holds at most 64 keys, one
-// wave ranks them directly (sel[4] must be zero on entry).  The caller passes a barrier before
-// sel, hist or sh is written again.
+// many of the keys equal to it fall within the need largest.  Histogram windows over the keys' range
+// (not their common prefix: 1.9 and 2.1 differ in the top bit), then over the chosen bin; once that
+// holds at most 64 keys, one wave ranks them directly (sel[4] must be zero on entry).  The caller
+// passes a barrier before sel, hist or sh is written again.
 DSA_DEV void select_exact(const uint32_t* keys, int m, int need, uint32_t lo, uint32_t hi, int* hist, int* sh,
                           int* sel, uint32_t& thr, int& need_out) {
   constexpr int T = kTopkThreads;
-  int pb = lo == hi ? 32 : __clz(lo ^ hi);              // bits shared by every key
-  uint32_t prefix = pb >= 32 ? lo : (pb == 0 ? 0u : lo & ~(0xFFFFFFFFu >> pb));
-  while (pb < 32) {
-    const int hi_shift = 32 - pb, shift = max(0, hi_shift - 11);
+  uint32_t last = hi - lo;
+  while (last > 0) {
+    const int shift = window_shift(last);
     int above, in_bin;
-    const int bin = window_pass(keys, m, prefix, hi_shift, shift, need, hist, sh, sel, &above, &in_bin);
-    prefix |= (uint32_t)bin << shift;
+    lo += (uint32_t)window_pass(keys, m, lo, last, shift, need, hist, sh, sel, &above, &in_bin) << shift;
+    last = (1u << shift) - 1;
     need -= above;
-    pb = 32 - shift;
-    if (pb < 32 && in_bin <= 64) {
+    if (last > 0 && in_bin <= 64) {
       // the bin's keys into hist[0..63] (slots from sel[4], zero on entry), then one wave ranks
       // them
       for (int i = threadIdx.x; i < m; i += T) {
         const uint32_t u = keys[i];
-        if (under_prefix(u, prefix, 32 - pb)) hist[atomicAdd(&sel[4], 1)] = (int)u;
+        if (u - lo <= last) hist[atomicAdd(&sel[4], 1)] = (int)u;
       }
       __syncthreads();
       if (threadIdx.x < 64) {
@@ -998,13 +991,11 @@ DSA_DEV void select_exact(const uint32_t* keys, int m, int need, uint32_t lo, ui
         const bool ok = l < in_bin;
         const uint32_t v = ok ? (uint32_t)hist[l] : 0u;
         int gt = 0, ge = 0;
-#pragma unroll 8
-        for (int j = 0; j < 64; ++j) {
+        const int n_bin = __builtin_amdgcn_readfirstlane(in_bin);
+        for (int j = 0; j < n_bin; ++j) {
           const uint32_t w = (uint32_t)__builtin_amdgcn_readlane((int)v, j);
-          if (j < in_bin) {
-            gt += w > v ? 1 : 0;
-            ge += w >= v ? 1 : 0;
-          }
+          gt += w > v ? 1 : 0;
+          ge += w >= v ? 1 : 0;
         }
         if (ok && gt < need && need <= ge) {   // every such lane holds the same key
           sel[1] = (int)v;
@@ -1017,7 +1008,7 @@ DSA_DEV void select_exact(const uint32_t* keys, int m, int need, uint32_t lo, ui
       return;
     }
   }
-  thr = prefix;
+  thr = lo;
   need_out = need;
 }
 
@@ -1029,8 +1020,7 @@ DSA_DEV void select_exact(const uint32_t* keys, int m, int need, uint32_t lo, ui
 //      r = ceil(1.5 K M / n) + 8 of the sample reach (the lower edge of the bin holding the
 //      sample's r-th largest), i.e. about 1.5 K of the row's entries;
 //   2  one pass over the row: every entry at or above the bound goes to an LDS candidate list with
-//      its position (wave-aggregated slots: counts bit-sliced over ballots, one LDS atomic per
-//      wave and step);
+//      its position (slots from ballots, one LDS atomic per wave and step);
 //   3  if the list holds between K and `cap` entries, it contains the whole top-K: the exact K-th
 //      largest key thr is selected over the candidates alone (select_exact), the selected
 //      positions (keys above thr, then the lowest-positioned `need` of the keys equal to it) are
@@ -1081,12 +1071,22 @@ DSA_DEV bool block_select_topk_sampled(const float* src, int n, int K, uint32_t*
     sel[3] = 0;
     sel[4] = 0;
   }
-  // ---- 1: sample keys, min / max, one window -> bound (workgroup-uniform)
+  // entries of the collect's next step, -0 past the row; the first step's are in flight under the bound
+  uint4 ahead[4];
+  auto load_step = [&](int g0) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int g = g0 + k * T + (int)threadIdx.x;
+      ahead[k] = g < n4 ? b4[g] : uint4{0x80000000u, 0x80000000u, 0x80000000u, 0x80000000u};
+    }
+  };
+  // ---- 1: sample keys, min / max, windows -> bound (workgroup-uniform)
   uint32_t bound;
   {
     const int run = threadIdx.x >> 3, part = threadIdx.x & 7;
     const int start = (int)(((int64_t)run * (n - 32) / 63) & ~3LL);   // + 31 < n
     const uint4 sv = b4[(start >> 2) + part];
+    load_step(0);
     const uint32_t s4[4] = {order_key(__builtin_bit_cast(float, sv.x)), order_key(__builtin_bit_cast(float, sv.y)),
                             order_key(__builtin_bit_cast(float, sv.z)), order_key(__builtin_bit_cast(float, sv.w))};
     *reinterpret_cast<uint4*>(ckey + 4 * threadIdx.x) = uint4{s4[0], s4[1], s4[2], s4[3]};
@@ -1094,66 +1094,69 @@ DSA_DEV bool block_select_topk_sampled(const float* src, int n, int K, uint32_t*
     uint32_t smin, smax;
     block_minmax(min(min(s4[0], s4[1]), min(s4[2], s4[3])), max(max(s4[0], s4[1]), max(s4[2], s4[3])), sh, smin,
                  smax);
+    // windows over the sample's range, until at most 1/16 of the r lie in the bin (scores of both signs:
+    // the first window's bins are a quarter of an octave, up to 1.6 times the candidates)
     bound = smin;
     if (smin != smax) {
-      const int hi_shift = 32 - __clz(smin ^ smax), shift = max(0, hi_shift - 11);
-      int above, in_bin;
-      const int bin = window_pass(ckey, M, smin, hi_shift, shift, r, hist, sh, sel, &above, &in_bin);
-      bound = (hi_shift >= 32 ? 0u : (smin >> hi_shift) << hi_shift) | ((uint32_t)bin << shift);
+      uint32_t last = smax - smin;
+      int want = r;
+      while (true) {
+        const int shift = window_shift(last);
+        int above, in_bin;
+        bound += (uint32_t)window_pass(ckey, M, bound, last, shift, want, hist, sh, sel, &above, &in_bin) << shift;
+        if (shift == 0 || 16 * in_bin <= r + 16) break;
+        want -= above;
+        last = (1u << shift) - 1;
+      }
     } else {
       __syncthreads();   // (block_minmax's reads of sh before the collect writes it)
     }
   }
 
   // ---- 2: candidates (keys >= bound) with their positions, 16 entries per thread and step
+  // (a workgroup's VALU bounds this step, 1.8 us per 8192 entries, 2.7 with order_key on all and a slot
+  // counted per lane: keys above a positive bound are the entries' bits with the sign flipped, and
+  // ballots give the slots)
+  bound = max(bound, 1u);   // 0: past the row
+  const bool flip = bound > 0x80000000u;
   uint32_t cmax = 0u;
   for (int g0 = 0; g0 < n4; g0 += 4 * T) {
-    uint4 x[4];
+    uint32_t e[16];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const int g = g0 + k * T + (int)threadIdx.x;
-      x[k] = g < n4 ? b4[g] : uint4{0u, 0u, 0u, 0u};   // past the row: never counted (ok below)
+      const uint4 x = ahead[k];
+      e[4 * k] = x.x; e[4 * k + 1] = x.y; e[4 * k + 2] = x.z; e[4 * k + 3] = x.w;
     }
-    int c = 0;
+    load_step(g0 + 4 * T);
+    if (flip) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const bool ok = g0 + k * T + (int)threadIdx.x < n4;
-      x[k] = uint4{order_key(__builtin_bit_cast(float, x[k].x)), order_key(__builtin_bit_cast(float, x[k].y)),
-                   order_key(__builtin_bit_cast(float, x[k].z)), order_key(__builtin_bit_cast(float, x[k].w))};
-      const uint32_t e[4] = {x[k].x, x[k].y, x[k].z, x[k].w};
+      for (int i = 0; i < 16; ++i) e[i] ^= 0x80000000u;
+    } else {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const bool in = ok && e[q] >= bound;
-        c += in ? 1 : 0;
-        cmax = in ? max(cmax, e[q]) : cmax;
-      }
+      for (int i = 0; i < 16; ++i)
+        e[i] = g0 + (i >> 2) * T + (int)threadIdx.x < n4 ? order_key(__builtin_bit_cast(float, e[i])) : 0u;
     }
-    // lane prefix of c over the wave from 5 bit-slice ballots (c <= 16)
-    int pre = 0, tot = 0;
+    uint64_t in[16];
+    int tot = 0;
 #pragma unroll
-    for (int bt = 0; bt < 5; ++bt) {
-      const uint64_t bm = __ballot((c >> bt) & 1);
-      pre += __popcll(bm & lt) << bt;
-      tot += __popcll(bm) << bt;
+    for (int i = 0; i < 16; ++i) {
+      cmax = max(cmax, e[i]);
+      in[i] = __ballot(e[i] >= bound);
+      tot += __popcll(in[i]);
     }
     if (tot == 0) continue;   // wave-uniform
     int slot0 = 0;
     if (lane == 0) slot0 = atomicAdd(&sel[3], tot);
-    int slot = __builtin_amdgcn_readfirstlane(slot0) + pre;
+    int base = __builtin_amdgcn_readfirstlane(slot0);
+    if (base + tot > cap) continue;   // (the count tells)
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int g = g0 + k * T + (int)threadIdx.x;
-      const uint32_t e[4] = {x[k].x, x[k].y, x[k].z, x[k].w};
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        if (g < n4 && e[q] >= bound) {
-          if (slot < cap) {
-            ckey[slot] = e[q];
-            cpos[slot] = (uint16_t)(4 * g + q);
-          }
-          ++slot;
-        }
+    for (int i = 0; i < 16; ++i) {
+      const int slot = __builtin_amdgcn_mbcnt_hi((uint32_t)(in[i] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)in[i], base));
+      if (e[i] >= bound) {
+        ckey[slot] = e[i];
+        cpos[slot] = (uint16_t)(4 * (g0 + (i >> 2) * T + (int)threadIdx.x) + (i & 3));
       }
+      base += __popcll(in[i]);
     }
   }
   for (int j = 4 * n4 + (int)threadIdx.x; j < n; j += T) {   // ragged tail (< 4 entries)
@@ -1508,17 +1511,19 @@ __global__ __launch_bounds__(kTopkThreads) void topk_merge_kernel(TopkParams p) 
 }
 #undef DSA_TOPK_SHARED
 
-// Split selection: fewer rows than this leave CUs idle in one-workgroup-per-row selection.
-// 16384-key slices (the LDS-cached length) beat 8192 at cfg5 decode: 47 vs 54 us, the merge then
-// taking half the candidates.
+// Split selection of fewer rows than this, which leave CUs idle in one-workgroup-per-row selection, from
+// the length on that one workgroup's sampled selection does not take.  It is the better one below:
+// 64 rows of 65532 keys, K = 2048, 29 us against 58 in slices of 16384 and a merge, of 32000 keys 19
+// against 46.  (The workspace is sized for slices of 16384.)
 constexpr int kTopkSplitRows = 256;
-constexpr int kTopkSliceMin = 16384;
+constexpr int kTopkSliceMin = kSampledMaxN;
+constexpr int kTopkWsSlice = 16384;
 
-int topk_slice_len(int topk) { return max(kTopkSliceMin, (topk + 3) / 4 * 16); }
+int topk_slice_len(int topk, int least) { return max(least, (topk + 3) / 4 * 16); }
 
 size_t topk_workspace_size(int rows, int64_t pitch, int topk) {
   if (rows <= 0 || rows >= kTopkSplitRows || topk < 1) return 0;
-  const int64_t slice = topk_slice_len(topk);
+  const int64_t slice = topk_slice_len(topk, kTopkWsSlice);
   if (pitch <= slice) return 0;
   const int64_t n_slices = (pitch + slice - 1) / slice;
   return (size_t)rows * n_slices * topk * (sizeof(uint32_t) + sizeof(int32_t));
@@ -1544,8 +1549,8 @@ int launch_topk(const TopkParams& p_in, hipStream_t stream) {
   if (p_in.rows == 0) return 0;
   TopkParams p = p_in;
   auto cache_for = [&](int64_t n) { return topk_cache_elems(n, p.topk); };
-  if (p.cand_key && topk_workspace_size(p.rows, p.pitch, p.topk) > 0) {
-    p.slice = topk_slice_len(p.topk);
+  p.slice = topk_slice_len(p.topk, kTopkSliceMin);
+  if (p.cand_key && topk_workspace_size(p.rows, p.pitch, p.topk) > 0 && p.pitch > p.slice) {
     p.n_slices = (int)((p.pitch + p.slice - 1) / p.slice);
     // rows up to one slice run whole in the slice kernel: its cache covers min(pitch, slice)
     p.cache_elems = cache_for(std::min<int64_t>(p.pitch, p.slice));

@@ -126,6 +126,34 @@ def test_topk_sampled_threshold_rows_bit_exact(case, n, k):
         assert torch.equal(got[r], ref), r
 
 
+@pytest.mark.parametrize("case", ["negative", "around_two", "zeros", "infinities"])
+@pytest.mark.parametrize("n,k", [(4096, 1), (4099, 900), (16385, 2048), (65535, 2048), (65537, 2048)])
+def test_topk_bound_and_windows_bit_exact(case, n, k):
+    """Where the sampled selection's bound and its histogram windows change form: scores without a
+    positive one, scores whose keys differ in the top exponent bit, a threshold among zeros of both
+    signs, infinities; at rows around its shortest and longest length and one past (slices).  Exact."""
+    print(f"[topk bound] case={case} n={n} k={k}", flush=True)
+    g = torch.Generator().manual_seed(n + k + len(case))
+    rows = 5
+    sc = torch.randn(rows, n, generator=g)
+    if case == "negative":
+        sc = -sc.abs() - 0.01
+    elif case == "around_two":
+        sc = 2.0 + 0.05 * sc
+    elif case == "zeros":
+        sc = torch.where(sc > 1.5, sc, torch.where(sc > 0, torch.zeros_like(sc), -torch.zeros_like(sc)))
+    else:
+        sc[:, ::97] = float("inf")
+        sc[:, 1::5] = float("-inf")
+    ln = torch.tensor([n, n - 1, n - 2, max(k, n - 1000), k], dtype=torch.int32)
+    base = torch.randint(0, 1000, (rows,), generator=g).to(torch.int32)
+    got = ops.topk(sc.to(DEV), base.to(DEV), ln.to(DEV), k).cpu().long()
+    for r in range(rows):
+        row = sc[r, :int(ln[r])].double()
+        order = torch.sort(row, descending=True, stable=True).indices[:k].sort().values   # ties: lower key
+        assert torch.equal(got[r], order + int(base[r])), r
+
+
 def test_topk_split_equals_one_workgroup_cfg5_full_size():
     """cfg5's 64 cache lengths (up to 65,265 keys): the split selection (slices + merge, through
     the workspace) returns the one-workgroup-per-row selection's indices bit for bit, on scores
