@@ -9,7 +9,9 @@ Megatron-compatible call signatures (sbhd layouts, ``fused_qk_topk_naive``) are 
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
+import functools
 from typing import Optional, Tuple
 
 import torch
@@ -21,12 +23,53 @@ D_QK = 576
 D_V = 512
 
 
+# (the entry points' argument types turn integers and None into pointers; a current-device guard and a
+# Stream object per call cost 3 us, as long as a launch)
 def _p(t: Optional[Tensor]):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
+    return t.data_ptr() if t is not None else None
 
 
 def _stream(dev: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(dev.index)
+
+
+_HERE = contextlib.nullcontext()
+
+
+def _on(dev: torch.device):
+    return _HERE if dev.index == torch._C._cuda_getDevice() else torch.cuda.device(dev)
+
+
+_LIBRARY = torch.library.Library("dsa_amd", "FRAGMENT")
+
+
+def _op(name: str, differentiable: bool = False):
+    """Registers a function as ``dsa_amd::name`` with the dispatcher, as ``torch.library.custom_op`` does,
+    which runs several Python layers around every call: 19 us a call, where the kernels of a short
+    prompt or of one decoded token take 10.  Where no input requires a gradient the call goes below the
+    autograd key, past the Python kernel there: 13 us with the launches' host side.  Tracing, fake tensors and function transforms
+    see the same op.  Without a formula (``differentiable``: the caller registers one) a backward
+    raises."""
+    def wrap(fn):
+        _LIBRARY.define(name + torch.library.infer_schema(fn, mutates_args=()), tags=(torch.Tag.pt2_compliant_tag,))
+        _LIBRARY.impl(name, fn, "CompositeExplicitAutograd")
+        overload = getattr(getattr(torch.ops.dsa_amd, name), "default")
+        if not differentiable:
+            def no_formula(ctx, *grads):
+                raise RuntimeError(f"Trying to backward through {overload} but no autograd formula was registered. "
+                                   "Please use register_autograd to add one.")
+            torch.library.register_autograd(f"dsa_amd::{name}", no_formula, lib=_LIBRARY)
+
+        @functools.wraps(fn)
+        def call(*args, **kwargs):
+            if torch.compiler.is_compiling() or (torch.is_grad_enabled() and torch._C._any_requires_grad(*args, **kwargs)):
+                return overload(*args, **kwargs)
+            with torch._C._AutoDispatchBelowAutograd():
+                return overload(*args, **kwargs)
+
+        call.register_fake = lambda fake: torch.library.register_fake(f"dsa_amd::{name}", fake, lib=_LIBRARY)
+        return call
+    return wrap
 
 
 def _require_gpu(*ts: Optional[Tensor]) -> None:
@@ -43,14 +86,14 @@ def _require(cond: bool, msg: str) -> None:
 # --------------------------------------------------------------------------------------
 # row descriptors (documents -> per-query visible key ranges)
 # --------------------------------------------------------------------------------------
-@torch.library.custom_op("dsa_amd::build_rows", mutates_args=())
+@_op("build_rows")
 def build_rows(cu_seqlens: Tensor, total_q: int, causal: bool) -> Tuple[Tensor, Tensor]:
     """Per-token ``(row_base, row_len)`` int32 from ``cu_seqlens`` (int32, on the GPU)."""
     _require_gpu(cu_seqlens)
     cu = cu_seqlens.to(torch.int32).contiguous()
     base = torch.empty(total_q, dtype=torch.int32, device=cu.device)
     ln = torch.empty(total_q, dtype=torch.int32, device=cu.device)
-    with torch.cuda.device(cu.device):
+    with _on(cu.device):
         _lib.call("dsa_build_rows", _p(cu), cu.numel() - 1, total_q, int(causal), _p(base), _p(ln), _stream(cu.device))
     return base, ln
 
@@ -63,7 +106,7 @@ def _(cu_seqlens, total_q, causal):
 # --------------------------------------------------------------------------------------
 # K0 indexer prologue
 # --------------------------------------------------------------------------------------
-@torch.library.custom_op("dsa_amd::indexer_prologue", mutates_args=())
+@_op("indexer_prologue", differentiable=True)
 def indexer_prologue(q_lin: Tensor, k_lin: Tensor, w_lin: Tensor, ln_weight: Tensor, ln_bias: Tensor,
                      freqs: Tensor, eps: float, mscale: float, deinterleave: bool, rotary_interleaved: bool,
                      fp8: bool = False) -> Tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
@@ -100,7 +143,7 @@ def indexer_prologue(q_lin: Tensor, k_lin: Tensor, w_lin: Tensor, ln_weight: Ten
     w = torch.empty(T, Hi, dtype=torch.float32, device=q_lin.device)
     qs = torch.empty((T, Hi) if fp8 else (0,), dtype=torch.float32, device=q_lin.device)
     ks = torch.empty((T,) if fp8 else (0,), dtype=torch.float32, device=q_lin.device)
-    with torch.cuda.device(q_lin.device):
+    with _on(q_lin.device):
         _lib.call("dsa_indexer_prologue", _p(q3), q3.stride(0), _p(kl), kl.stride(0), _p(wl), wl.stride(0),
                   _p(lw), _p(lb), _p(fr), fr.stride(0), T, Hi, 128, 64, float(eps), float(mscale),
                   float(Hi ** -0.5), float(128 ** -0.5), int(deinterleave), int(rotary_interleaved),
@@ -119,7 +162,7 @@ def _(q_lin, k_lin, w_lin, ln_weight, ln_bias, freqs, eps, mscale, deinterleave,
             q_lin.new_empty(T, Hi, dtype=torch.float32))
 
 
-@torch.library.custom_op("dsa_amd::indexer_prologue_bwd", mutates_args=())
+@_op("indexer_prologue_bwd")
 def indexer_prologue_bwd(dq: Tensor, dk: Tensor, dw: Tensor, k_lin: Tensor, ln_weight: Tensor, freqs: Tensor,
                          eps: float, mscale: float, deinterleave: bool,
                          rotary_interleaved: bool) -> Tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
@@ -142,7 +185,7 @@ def indexer_prologue_bwd(dq: Tensor, dk: Tensor, dw: Tensor, k_lin: Tensor, ln_w
     dlb = torch.empty(128, dtype=torch.float32, device=dev)
     ws_bytes = int(_lib.load().dsa_indexer_prologue_bwd_workspace_size(T))
     ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call("dsa_indexer_prologue_bwd", _p(dq), _p(dk), _p(dw), _p(kl), kl.stride(0), _p(lw), _p(fr),
                   fr.stride(0), T, Hi, 128, 64, float(eps), float(mscale), float(Hi ** -0.5), float(128 ** -0.5),
                   int(deinterleave), int(rotary_interleaved), _p(dq_lin), Hi * 128, _p(dk_lin), 128, _p(dw_lin), Hi,
@@ -182,13 +225,13 @@ def _pro_backward(ctx, dq, dqs, dk, dks, dw):
             None, None, None, None, None, None)
 
 
-torch.library.register_autograd("dsa_amd::indexer_prologue", _pro_backward, setup_context=_pro_setup)
+torch.library.register_autograd("dsa_amd::indexer_prologue", _pro_backward, setup_context=_pro_setup, lib=_LIBRARY)
 
 
 # --------------------------------------------------------------------------------------
 # K1 indexer scores
 # --------------------------------------------------------------------------------------
-@torch.library.custom_op("dsa_amd::indexer_scores", mutates_args=())
+@_op("indexer_scores", differentiable=True)
 def indexer_scores(q: Tensor, k: Tensor, w: Tensor, row_base: Tensor, row_len: Tensor, max_row_len: int,
                    pitch: int, q_scale: Optional[Tensor] = None, k_scale: Optional[Tensor] = None,
                    fill_masked: bool = False) -> Tensor:
@@ -210,7 +253,7 @@ def indexer_scores(q: Tensor, k: Tensor, w: Tensor, row_base: Tensor, row_len: T
     ks = k_scale.to(torch.float32).contiguous() if fp8 else None
     scores = torch.empty(T, pitch, dtype=torch.float32, device=q.device)
     dt = _lib.DSA_FP8_E4M3 if fp8 else _lib.DSA_BF16
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         _lib.call("dsa_indexer_scores", _p(q), dt, _p(qs), _p(k), dt, _p(ks), _p(w), _p(row_base.contiguous()),
                   _p(row_len.contiguous()), T, k.shape[0], Hi, Di, max_row_len, _p(scores), pitch,
                   int(fill_masked), _stream(q.device))
@@ -225,7 +268,7 @@ def _(q, k, w, row_base, row_len, max_row_len, pitch, q_scale=None, k_scale=None
 # --------------------------------------------------------------------------------------
 # K2 top-k
 # --------------------------------------------------------------------------------------
-@torch.library.custom_op("dsa_amd::topk", mutates_args=())
+@_op("topk")
 def topk(scores: Tensor, row_base: Tensor, row_len: Tensor, k: int) -> Tensor:
     """Per row the ``min(k, row_len)`` largest scores (ties -> lower key) as ascending key ids
     ``row_base + j``, ``-1`` padded.  int32 ``[rows, k]``."""
@@ -237,7 +280,7 @@ def topk(scores: Tensor, row_base: Tensor, row_len: Tensor, k: int) -> Tensor:
     # few long rows (decode) split each row over several workgroups through this workspace
     nws = int(_lib.load().dsa_topk_workspace_size(rows, s.stride(0), k))
     ws = torch.empty(max(nws, 1), dtype=torch.uint8, device=s.device)
-    with torch.cuda.device(s.device):
+    with _on(s.device):
         _lib.call("dsa_topk", _p(s), s.stride(0), _p(row_base.contiguous()), _p(row_len.contiguous()), rows, k,
                   _p(out), ctypes.c_void_p(0), _p(ws) if nws else ctypes.c_void_p(0), nws, _stream(s.device))
     return out
@@ -267,7 +310,7 @@ def indexer_topk(q: Tensor, k: Tensor, w: Tensor, index_topk: int, cu_seqlens: O
     return (idx, sc) if return_scores else idx
 
 
-@torch.library.custom_op("dsa_amd::build_decode_rows", mutates_args=())
+@_op("build_decode_rows")
 def build_decode_rows(cu_cache: Tensor) -> Tuple[Tensor, Tensor]:
     """Per-sequence ``(row_base, row_len)`` int32 of one new token per sequence over its whole
     cache: ``row_base[b] = cu_cache[b]``, ``row_len[b] = cu_cache[b+1] - cu_cache[b]``."""
@@ -276,7 +319,7 @@ def build_decode_rows(cu_cache: Tensor) -> Tuple[Tensor, Tensor]:
     B = cu.numel() - 1
     base = torch.empty(B, dtype=torch.int32, device=cu.device)
     ln = torch.empty(B, dtype=torch.int32, device=cu.device)
-    with torch.cuda.device(cu.device):
+    with _on(cu.device):
         _lib.call("dsa_build_decode_rows", _p(cu), B, _p(base), _p(ln), _stream(cu.device))
     return base, ln
 
@@ -316,7 +359,7 @@ def _check_attn(q: Tensor, kv: Tensor, idx: Tensor, q512: bool = False) -> None:
     _require(q.dtype == torch.bfloat16 and kv.dtype == torch.bfloat16, "q and kv must be bf16")
 
 
-@torch.library.custom_op("dsa_amd::sparse_mla_fwd", mutates_args=())
+@_op("sparse_mla_fwd", differentiable=True)
 def sparse_mla_fwd(q: Tensor, kv: Tensor, idx: Tensor, sm_scale: float, causal: bool = False) -> Tuple[Tensor, Tensor]:
     """Absorbed sparse MLA forward: ``(out [T,H,512] bf16, lse [T,H] fp32)``."""
     _check_attn(q, kv, idx)
@@ -326,7 +369,7 @@ def sparse_mla_fwd(q: Tensor, kv: Tensor, idx: Tensor, sm_scale: float, causal: 
     T, H, _ = q.shape
     out = torch.empty(T, H, D_V, dtype=torch.bfloat16, device=q.device)
     lse = torch.empty(T, H, dtype=torch.float32, device=q.device)
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         _lib.call("dsa_sparse_mla_fwd", _p(q), _p(kv), _p(idx), T, kv.shape[0], H, D_QK, D_V, idx.shape[1],
                   float(sm_scale), int(causal), _p(out), _p(lse), _stream(q.device))
     return out, lse
@@ -338,7 +381,7 @@ def _(q, kv, idx, sm_scale, causal=False):
     return q.new_empty(T, H, D_V), q.new_empty(T, H, dtype=torch.float32)
 
 
-@torch.library.custom_op("dsa_amd::sparse_mla_fwd_sink", mutates_args=())
+@_op("sparse_mla_fwd_sink")
 def sparse_mla_fwd_sink(q: Tensor, kv: Tensor, idx: Tensor, sinks: Tensor, sm_scale: float,
                         causal: bool = False) -> Tuple[Tensor, Tensor]:
     """``sparse_mla_fwd`` with a per-head attention sink ``sinks [H]`` (a logit with no value row):
@@ -354,7 +397,7 @@ def sparse_mla_fwd_sink(q: Tensor, kv: Tensor, idx: Tensor, sinks: Tensor, sm_sc
     _require(sk.shape == (H,), "sinks must be [H]")
     out = torch.empty(T, H, D_V, dtype=torch.bfloat16, device=q.device)
     lse = torch.empty(T, H, dtype=torch.float32, device=q.device)
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         _lib.call("dsa_sparse_mla_fwd_sink", _p(q), _p(kv), _p(idx), T, kv.shape[0], H, q.shape[-1], D_V,
                   idx.shape[1], float(sm_scale), int(causal), _p(sk), _p(out), _p(lse), _stream(q.device))
     return out, lse
@@ -366,7 +409,7 @@ def _(q, kv, idx, sinks, sm_scale, causal=False):
     return q.new_empty(T, H, D_V), q.new_empty(T, H, dtype=torch.float32)
 
 
-@torch.library.custom_op("dsa_amd::sparse_mla_bwd_sink", mutates_args=())
+@_op("sparse_mla_bwd_sink")
 def sparse_mla_bwd_sink(q: Tensor, kv: Tensor, idx: Tensor, out: Tensor, dout: Tensor, lse: Tensor, sinks: Tensor,
                         sm_scale: float, causal: bool = False) -> Tuple[Tensor, Tensor, Tensor]:
     """Gradients of ``sparse_mla_fwd_sink`` from its ``out`` and ``lse``: ``(dq`` (bf16, the shape of
@@ -392,7 +435,7 @@ def sparse_mla_bwd_sink(q: Tensor, kv: Tensor, idx: Tensor, out: Tensor, dout: T
         dbytes = (T * H * 4 + 255) // 256 * 256
         ws_bytes = max(cap, bwd_workspace_bytes_chunked(T, N, H, K, 256, g_int8) + dbytes)
     ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=q.device)
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         _lib.call("dsa_sparse_mla_bwd_sink", _p(q), _p(kv), _p(idx), _p(out), _p(dout), _p(lse), _p(sk), T, N, H,
                   q.shape[-1], D_V, K, float(sm_scale), int(causal), _p(dq), _p(dkv), _p(dsk), flags, _p(ws), ws.numel(),
                   _stream(q.device))
@@ -409,7 +452,7 @@ def decode_workspace_bytes(batch: int, n_heads: int, topk_: int) -> int:
     return int(_lib.load().dsa_sparse_mla_decode_workspace_size(batch, n_heads, topk_))
 
 
-@torch.library.custom_op("dsa_amd::sparse_mla_decode", mutates_args=())
+@_op("sparse_mla_decode")
 def sparse_mla_decode(q: Tensor, kv_cache: Tensor, idx: Tensor, sm_scale: float) -> Tuple[Tensor, Tensor]:
     """Decode attention of one new token per sequence: ``q [B,H,576]`` over its selected rows
     of ``kv_cache [N,576]`` (``idx [B,K]`` global rows).  ``(out [B,H,512] bf16, lse [B,H])``."""
@@ -423,7 +466,7 @@ def sparse_mla_decode(q: Tensor, kv_cache: Tensor, idx: Tensor, sm_scale: float)
     lse = torch.empty(B, H, dtype=torch.float32, device=q.device)
     ws_bytes = decode_workspace_bytes(B, H, K)
     ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=q.device)
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         _lib.call("dsa_sparse_mla_decode", _p(q), _p(kv_cache), _p(idx), B, kv_cache.shape[0], H, D_QK, D_V, K,
                   float(sm_scale), _p(out), _p(lse), _p(ws), ws_bytes, _stream(q.device))
     return out, lse
@@ -450,7 +493,7 @@ def bwd_workspace_bytes_chunked(total_q: int, n_kv: int, n_heads: int, topk_: in
                                                                  flags))
 
 
-@torch.library.custom_op("dsa_amd::sparse_mla_bwd", mutates_args=())
+@_op("sparse_mla_bwd")
 def sparse_mla_bwd(q: Tensor, kv: Tensor, idx: Tensor, out: Tensor, dout: Tensor, lse: Tensor, sm_scale: float,
                    causal: bool = False, max_workspace_bytes: int = 0, g_int8: bool = False) -> Tuple[Tensor, Tensor]:
     """Gradients of ``sparse_mla_fwd``: ``(dq [T,H,576] bf16, dkv [N,576] fp32)``.
@@ -474,7 +517,7 @@ def sparse_mla_bwd(q: Tensor, kv: Tensor, idx: Tensor, out: Tensor, dout: Tensor
     if 0 < cap < ws_bytes:
         ws_bytes = max(cap, bwd_workspace_bytes_chunked(T, N, H, K, 256, g_int8))
     ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=q.device)
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         _lib.call("dsa_sparse_mla_bwd_ex", _p(q), _p(kv), _p(idx), _p(out), _p(dout), _p(lse), T, N, H, D_QK, D_V,
                   K, float(sm_scale), int(causal), _p(dq), _p(dkv), DSA_BWD_G_INT8 if g_int8 else 0, _p(ws),
                   ws_bytes, None, _stream(q.device))
@@ -486,7 +529,7 @@ def _(q, kv, idx, out, dout, lse, sm_scale, causal=False, max_workspace_bytes=0,
     return torch.empty_like(q), kv.new_empty(kv.shape[0], D_QK, dtype=torch.float32)
 
 
-@torch.library.custom_op("dsa_amd::sparse_mla_bwd_with_target", mutates_args=())
+@_op("sparse_mla_bwd_with_target")
 def sparse_mla_bwd_with_target(q: Tensor, kv: Tensor, idx: Tensor, out: Tensor, dout: Tensor, lse: Tensor,
                                sm_scale: float, causal: bool = False) -> Tuple[Tensor, Tensor, Tensor]:
     """``sparse_mla_bwd`` plus the sparse indexer loss target ``[T, K]`` fp32, read from the P tiles
@@ -503,7 +546,7 @@ def sparse_mla_bwd_with_target(q: Tensor, kv: Tensor, idx: Tensor, out: Tensor, 
     tgt = torch.empty(T, K, dtype=torch.float32, device=q.device)
     ws_bytes = bwd_workspace_bytes(T, N, H, K)
     ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=q.device)
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         _lib.call("dsa_sparse_mla_bwd", _p(q), _p(kv), _p(idx), _p(out), _p(dout), _p(lse), T, N, H, D_QK, D_V, K,
                   float(sm_scale), int(causal), _p(dq), _p(dkv), _p(ws), ws_bytes, _stream(q.device))
         _lib.call("dsa_indexer_kl_target_from_bwd", _p(ws), ws_bytes, _p(idx), T, N, H, K, int(causal), _p(tgt),
@@ -597,7 +640,7 @@ def _fwd_backward(ctx, dout, dlse):
     return dq, dkv.to(kv.dtype), None, None, None
 
 
-torch.library.register_autograd("dsa_amd::sparse_mla_fwd", _fwd_backward, setup_context=_fwd_setup)
+torch.library.register_autograd("dsa_amd::sparse_mla_fwd", _fwd_backward, setup_context=_fwd_setup, lib=_LIBRARY)
 
 
 def sparse_mla(q: Tensor, kv: Tensor, idx: Tensor, sm_scale: float, causal: bool = False) -> Tensor:
@@ -608,7 +651,7 @@ def sparse_mla(q: Tensor, kv: Tensor, idx: Tensor, sm_scale: float, causal: bool
 # --------------------------------------------------------------------------------------
 # indexer KL loss: target, per-row KL + gradient, selected-slot scores and their backward
 # --------------------------------------------------------------------------------------
-@torch.library.custom_op("dsa_amd::indexer_kl_target", mutates_args=())
+@_op("indexer_kl_target")
 def indexer_kl_target(q: Tensor, kv: Tensor, idx: Tensor, lse: Tensor, sm_scale: float, causal: bool = True) -> Tensor:
     """Head-averaged attention probability of every selected key, ``[T, K]`` fp32 (0 at invalid
     slots), recomputed from the sparse forward's ``lse``: the target of the sparse indexer loss."""
@@ -619,7 +662,7 @@ def indexer_kl_target(q: Tensor, kv: Tensor, idx: Tensor, lse: Tensor, sm_scale:
     T, H, _ = q.shape
     _require(lse.shape == (T, H), "lse must be [T, H]")
     tgt = torch.empty(T, idx.shape[1], dtype=torch.float32, device=q.device)
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         _lib.call("dsa_indexer_kl_target", _p(q), _p(kv), _p(idx), _p(lse), T, kv.shape[0], H, D_QK, idx.shape[1],
                   float(sm_scale), int(causal), _p(tgt), _stream(q.device))
     return tgt
@@ -630,7 +673,7 @@ def _(q, kv, idx, lse, sm_scale, causal=True):
     return q.new_empty(q.shape[0], idx.shape[1], dtype=torch.float32)
 
 
-@torch.library.custom_op("dsa_amd::indexer_kl_rows", mutates_args=())
+@_op("indexer_kl_rows")
 def indexer_kl_rows(index_sel: Tensor, target: Tensor, idx: Tensor, n_kv: int, causal: bool,
                     grad_scale: float) -> Tuple[Tensor, Tensor]:
     """Per-query KL of the sparse indexer loss, ``kl [T]``, and ``grad_scale * d kl_t / d index_sel``
@@ -642,7 +685,7 @@ def indexer_kl_rows(index_sel: Tensor, target: Tensor, idx: Tensor, n_kv: int, c
     _require(index_sel.shape == (T, K) and target.shape == (T, K), "index_sel and target must be [T, K]")
     kl = torch.empty(T, dtype=torch.float32, device=idx.device)
     d = torch.empty(T, K, dtype=torch.float32, device=idx.device)
-    with torch.cuda.device(idx.device):
+    with _on(idx.device):
         _lib.call("dsa_indexer_kl_loss", _p(index_sel), _p(target), _p(idx), T, int(n_kv), K, int(causal),
                   float(grad_scale), _p(kl), _p(d), _stream(idx.device))
     return kl, d
@@ -662,7 +705,7 @@ def _check_idx_sel(q: Tensor, k: Tensor, w: Tensor, idx: Tensor) -> None:
     _require(idx.dim() == 2 and idx.shape[0] == q.shape[0], "idx must be [T, K]")
 
 
-@torch.library.custom_op("dsa_amd::indexer_selected_scores", mutates_args=())
+@_op("indexer_selected_scores", differentiable=True)
 def indexer_selected_scores(q: Tensor, k: Tensor, w: Tensor, idx: Tensor, causal: bool = True) -> Tensor:
     """Indexer scores of the selected slots, ``sum_h w[t,h] relu(q[t,h] . k[idx[t,j]])`` ``[T, K]``
     fp32 (-inf at invalid slots); differentiable in q, k and w."""
@@ -671,7 +714,7 @@ def indexer_selected_scores(q: Tensor, k: Tensor, w: Tensor, idx: Tensor, causal
     idx = idx.to(torch.int32).contiguous()
     T, Hi, _ = q.shape
     sc = torch.empty(T, idx.shape[1], dtype=torch.float32, device=q.device)
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         _lib.call("dsa_indexer_selected_scores", _p(q), _p(k), _p(w), _p(idx), T, k.shape[0], Hi, 128,
                   idx.shape[1], int(causal), _p(sc), _stream(q.device))
     return sc
@@ -686,7 +729,7 @@ def indexer_scores_bwd_workspace_bytes(total_q: int, n_k: int, topk_: int) -> in
     return int(_lib.load().dsa_indexer_scores_bwd_workspace_size(total_q, n_k, topk_))
 
 
-@torch.library.custom_op("dsa_amd::indexer_scores_bwd", mutates_args=())
+@_op("indexer_scores_bwd")
 def indexer_scores_bwd(q: Tensor, k: Tensor, w: Tensor, idx: Tensor, d_scores: Tensor,
                        causal: bool = True) -> Tuple[Tensor, Tensor, Tensor]:
     """Gradients of ``indexer_selected_scores``: ``(dq [T,Hi,128], dw [T,Hi], dk [N,128])`` fp32."""
@@ -703,7 +746,7 @@ def indexer_scores_bwd(q: Tensor, k: Tensor, w: Tensor, idx: Tensor, d_scores: T
     dk = torch.empty(N, 128, dtype=torch.float32, device=q.device)
     ws_bytes = indexer_scores_bwd_workspace_bytes(T, N, K)
     ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=q.device)
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         _lib.call("dsa_indexer_scores_bwd", _p(q), _p(k), _p(w), _p(idx), _p(d_scores), T, N, Hi, 128, K,
                   int(causal), _p(dq), _p(dw), _p(dk), _p(ws), ws_bytes, _stream(q.device))
     return dq, dw, dk
@@ -728,7 +771,7 @@ def _sel_backward(ctx, d_scores):
     return dq.to(q.dtype), dk.to(k.dtype), dw.to(w.dtype), None, None
 
 
-torch.library.register_autograd("dsa_amd::indexer_selected_scores", _sel_backward, setup_context=_sel_setup)
+torch.library.register_autograd("dsa_amd::indexer_selected_scores", _sel_backward, setup_context=_sel_setup, lib=_LIBRARY)
 
 
 # --------------------------------------------------------------------------------------
@@ -771,7 +814,7 @@ def indexer_scores_dense_bwd(q: Tensor, k: Tensor, w: Tensor, row_base: Tensor, 
     dk = torch.empty(N, 128, dtype=torch.float32, device=q.device)
     ws_bytes = dense_scores_bwd_workspace_bytes(T, N)
     ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=q.device)
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         _lib.call("dsa_dense_indexer_scores_bwd", _p(q), _p(k), _p(w), _p(rb), _p(rl), T, N, Hi, 128, _p(d),
                   d.shape[1], _p(dq), _p(dw), _p(dk), _p(ws), ws.numel(), _stream(q.device))
     return dq, dw, dk
@@ -792,7 +835,7 @@ def _isc_backward(ctx, d_scores):
     return dq.to(q.dtype), dk.to(k.dtype), dw.to(w.dtype), None, None, None, None, None, None, None
 
 
-torch.library.register_autograd("dsa_amd::indexer_scores", _isc_backward, setup_context=_isc_setup)
+torch.library.register_autograd("dsa_amd::indexer_scores", _isc_backward, setup_context=_isc_setup, lib=_LIBRARY)
 
 
 def _check_dense(q: Tensor, kv: Tensor, row_base: Tensor, row_len: Tensor) -> None:
@@ -816,7 +859,7 @@ def dense_attention_lse(q: Tensor, kv: Tensor, row_base: Tensor, row_len: Tensor
     if T == 0 or max_row_len <= 0:
         return lse.fill_(float("-inf"))
     rb, rl = row_base.to(torch.int32).contiguous(), row_len.to(torch.int32).contiguous()
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         _lib.call("dsa_dense_attention_lse", _p(q), _p(kv), _p(rb), _p(rl), T, kv.shape[0], H, D_QK,
                   float(sm_scale), _p(lse), _stream(q.device))
     return lse
@@ -836,7 +879,7 @@ def dense_attention_target(q: Tensor, kv: Tensor, lse: Tensor, row_base: Tensor,
         return tgt.zero_()
     rb, rl = row_base.to(torch.int32).contiguous(), row_len.to(torch.int32).contiguous()
     lse = lse.to(torch.float32).contiguous()
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         _lib.call("dsa_dense_attention_target", _p(q), _p(kv), _p(lse), _p(rb), _p(rl), T, kv.shape[0], H, D_QK,
                   int(pitch), float(sm_scale), _p(tgt), _stream(q.device))
     return tgt
@@ -900,7 +943,7 @@ def v4_compress_fwd(kv: Tensor, gate: Tensor, ape: Tensor, norm_w: Tensor, table
     T = kv.shape[0]
     ape, norm_w = ape.contiguous(), norm_w.contiguous()
     out = torch.empty(n_entries, D, dtype=torch.bfloat16, device=kv.device)
-    with torch.cuda.device(kv.device):
+    with _on(kv.device):
         _lib.call("dsa_v4_compress_fwd", _p(kv), _p(gate), kv.stride(0), gate.stride(0), _p(ape), _p(norm_w),
                   _p(table), table.shape[1] - 1, T, int(n_entries), C, D, int(rate), int(bool(overlap)), float(eps),
                   _p(out), _stream(kv.device))
@@ -922,7 +965,7 @@ def v4_compress_bwd(kv: Tensor, gate: Tensor, ape: Tensor, norm_w: Tensor, table
     dnorm = torch.empty(D, dtype=torch.float32, device=kv.device)
     ws_bytes = int(_lib.load().dsa_v4_compress_bwd_workspace_size(int(n_entries), int(n_items), C, D, int(rate)))
     ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=kv.device)
-    with torch.cuda.device(kv.device):
+    with _on(kv.device):
         _lib.call("dsa_v4_compress_bwd", _p(kv), _p(gate), kv.stride(0), gate.stride(0), _p(ape), _p(norm_w),
                   _p(table), table.shape[1] - 1, T, int(n_entries), int(n_items), C, D, int(rate),
                   int(bool(overlap)), float(eps), _p(dout), _p(dkv), _p(dgate), C, C, _p(dape), _p(dnorm), _p(ws),
@@ -953,7 +996,7 @@ def v4_norm_rope(x: Tensor, cos: Tensor, sin: Tensor, rope_dim: int, norm: bool,
     out = torch.empty_like(x)
     if out.numel() == 0:
         return out
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         _lib.call("dsa_v4_norm_rope", _p(x), T * H, H, D, int(rope_dim), _p(cos), _p(sin), cos.stride(0), int(bool(norm)),
                   float(eps), int(bool(inverse)), _p(out), _stream(x.device))
     return out
@@ -968,7 +1011,7 @@ def v4_norm_rope_bwd(x: Tensor, dout: Tensor, cos: Tensor, sin: Tensor, rope_dim
     dx = torch.empty_like(dout)
     if dx.numel() == 0:
         return dx
-    with torch.cuda.device(dout.device):
+    with _on(dout.device):
         _lib.call("dsa_v4_norm_rope_bwd", _p(x), _p(dout), T * H, H, D, int(rope_dim), _p(cos), _p(sin), cos.stride(0),
                   int(bool(norm)), float(eps), int(bool(inverse)), _p(dx), _stream(dout.device))
     return dx
@@ -981,7 +1024,7 @@ def v4_out_rope_group(o: Tensor, cos: Tensor, sin: Tensor, rope_dim: int, groups
     T, H, D = o.shape
     _require(H % groups == 0 and cos.shape[0] == T, "heads must split into the groups; one cos / sin row per token")
     og = torch.empty(groups, T, H * D // groups, dtype=o.dtype, device=o.device)
-    with torch.cuda.device(o.device):
+    with _on(o.device):
         _lib.call("dsa_v4_out_rope_group", _p(o), T, H, D, int(rope_dim), int(groups), _p(cos), _p(sin), cos.stride(0),
                   int(bool(inverse)), _p(og), _stream(o.device))
     return og
@@ -994,7 +1037,7 @@ def v4_out_rope_group_bwd(dog: Tensor, n_heads: int, cos: Tensor, sin: Tensor, r
     _require((W * G) % n_heads == 0, "the grouped rows must hold whole heads")
     D = W * G // n_heads
     d_o = torch.empty(T, n_heads, D, dtype=dog.dtype, device=dog.device)
-    with torch.cuda.device(dog.device):
+    with _on(dog.device):
         _lib.call("dsa_v4_out_rope_group_bwd", _p(dog), T, n_heads, D, int(rope_dim), G, _p(cos), _p(sin),
                   cos.stride(0), int(bool(inverse)), _p(d_o), _stream(dog.device))
     return d_o

@@ -3,6 +3,7 @@ mask-type / packing helpers of the Megatron-shaped drop-ins."""
 import sys
 import types
 
+import pytest
 import torch
 
 from mcore_bridge_amd import patch, dsa, workloads as W
@@ -259,3 +260,26 @@ def test_prologue_hadamard_lane_stages():
             neg = (((L ^ (L >> 1)) & (L >> 2)) ^ bin(L).count("1")) & 1
             want = np.array([[ref[64 * h + 4 * C + e] for e in range(4)] for h in range(2)])
             np.testing.assert_allclose(v[L] * (-1.0 if neg else 1.0), want, rtol=0, atol=1e-9)
+
+
+def test_ops_are_dispatcher_ops():
+    """The ops keep what a dispatcher op gives where a call skips the autograd key: fake tensors, traces
+    that record the op, refusal of CPU tensors, and a backward without a formula that raises."""
+    from torch._subclasses import FakeTensorMode
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from mcore_bridge_amd import ops
+    sc, ln = torch.zeros(2, 8), torch.zeros(2, dtype=torch.int32)
+    for s in (sc, sc.clone().requires_grad_()):
+        with pytest.raises(RuntimeError, match="run on the GPU"):
+            ops.topk(s, ln, ln, k=3)
+    g = make_fx(lambda s, n: ops.topk(s, n, n, 3), tracing_mode="fake")(sc, ln)
+    assert any(n.target is torch.ops.dsa_amd.topk.default for n in g.graph.nodes)
+    with FakeTensorMode():
+        q = torch.empty(2, 16, 576, dtype=torch.bfloat16, device="cuda", requires_grad=True)
+        kv, idx = torch.empty(9, 576, dtype=torch.bfloat16, device="cuda"), torch.empty(2, 4, dtype=torch.int32, device="cuda")
+        out, _ = ops.sparse_mla_decode(q, kv, idx, 0.1)
+        assert out.shape == (2, 16, 512) and out.requires_grad
+        with pytest.raises(RuntimeError, match="no autograd formula"):
+            out.sum().backward()
+        with torch.no_grad():
+            assert not ops.sparse_mla_decode(q, kv, idx, 0.1)[0].requires_grad
