@@ -47,9 +47,8 @@ def _op(name: str, differentiable: bool = False):
     """Registers a function as ``dsa_amd::name`` with the dispatcher, as ``torch.library.custom_op`` does,
     which runs several Python layers around every call: 19 us a call, where the kernels of a short
     prompt or of one decoded token take 10.  Where no input requires a gradient the call goes below the
-    autograd key, past the Python kernel there: 13 us with the launches' host side.  Tracing, fake tensors and function transforms
-    see the same op.  Without a formula (``differentiable``: the caller registers one) a backward
-    raises."""
+    autograd key, past the Python kernel there: 13 us.  Tracing, fake tensors and function transforms see
+    the same op.  Without a formula (``differentiable``: the caller registers one) a backward raises."""
     def wrap(fn):
         _LIBRARY.define(name + torch.library.infer_schema(fn, mutates_args=()), tags=(torch.Tag.pt2_compliant_tag,))
         _LIBRARY.impl(name, fn, "CompositeExplicitAutograd")

@@ -263,9 +263,8 @@ def test_prologue_hadamard_lane_stages():
 
 
 def test_ops_are_dispatcher_ops():
-    """The ops keep what a dispatcher op gives where a call skips the autograd key: fake tensors, traces
+    """The ops keep what a dispatcher op gives where a call skips the autograd key: meta tensors, traces
     that record the op, refusal of CPU tensors, and a backward without a formula that raises."""
-    from torch._subclasses import FakeTensorMode
     from torch.fx.experimental.proxy_tensor import make_fx
     from mcore_bridge_amd import ops
     sc, ln = torch.zeros(2, 8), torch.zeros(2, dtype=torch.int32)
@@ -274,12 +273,11 @@ def test_ops_are_dispatcher_ops():
             ops.topk(s, ln, ln, k=3)
     g = make_fx(lambda s, n: ops.topk(s, n, n, 3), tracing_mode="fake")(sc, ln)
     assert any(n.target is torch.ops.dsa_amd.topk.default for n in g.graph.nodes)
-    with FakeTensorMode():
-        q = torch.empty(2, 16, 576, dtype=torch.bfloat16, device="cuda", requires_grad=True)
-        kv, idx = torch.empty(9, 576, dtype=torch.bfloat16, device="cuda"), torch.empty(2, 4, dtype=torch.int32, device="cuda")
-        out, _ = ops.sparse_mla_decode(q, kv, idx, 0.1)
-        assert out.shape == (2, 16, 512) and out.requires_grad
-        with pytest.raises(RuntimeError, match="no autograd formula"):
-            out.sum().backward()
-        with torch.no_grad():
-            assert not ops.sparse_mla_decode(q, kv, idx, 0.1)[0].requires_grad
+    q = torch.empty(2, 16, 576, dtype=torch.bfloat16, device="meta", requires_grad=True)
+    kv, idx = torch.empty(9, 576, dtype=torch.bfloat16, device="meta"), torch.empty(2, 4, dtype=torch.int32, device="meta")
+    out, _ = ops.sparse_mla_decode(q, kv, idx, 0.1)
+    assert out.shape == (2, 16, 512) and out.requires_grad
+    with pytest.raises(RuntimeError, match="no autograd formula"):
+        out.sum().backward()
+    with torch.no_grad():
+        assert not ops.sparse_mla_decode(q, kv, idx, 0.1)[0].requires_grad
