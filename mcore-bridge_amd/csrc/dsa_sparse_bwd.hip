@@ -16,7 +16,7 @@
 // streaming pass instead.
 //   B1 bwd_sp_kernel   per query: recompute S, P, dP (shared K/V operand reads), Delta fused;
 //                      stage P and scale*dS (bf16 chunks of 32 keys x 16 heads, dsa_common.h).
-//   B2 bwd_dq_kernel   per query: dQ^T += K^T . dS^T over the gathered rows (K^T via transposing
+//   B2 bwd_dq8_kernel  per query: dQ^T += K^T . dS^T over the gathered rows (K^T via transposing
 //                      LDS reads, dS^T tile copied into LDS next to the KV tile).
 //   B3 bwd_g_kernel    per query: G^T[576 x keys] = Q^T . dS + dO^T . P contracted over all
 //                      heads (Q^T / dO^T held in registers), written as bf16 rows at the pair's
